@@ -568,11 +568,12 @@ struct StagePlan {
         uint64_t tiles = 0;
         uint64_t flops = 0;             // MFMA flops of the visited tiles (unpadded)
         bool narrow = true;             // every task's T_D step window fits 32-bit byte offsets
+        std::vector<uint32_t> tile_cols;   // per tile: the 16-column blocks holding a nonzero (bits)
         // per tile: its group, first key and first column: the dense W_D can be rebuilt from the
         // tiles (the flop model reads W_D; the device keeps only the tiles)
         struct TileAt { uint32_t group, k0, n0; };
         std::vector<TileAt> tile_at;
-        DevBuf d_tasks, d_runs, d_w64, d_w32, d_whi, d_wlo;
+        DevBuf d_tasks, d_runs, d_tile_cols, d_w64, d_w32, d_whi, d_wlo;
     } bsr;
     bool bsr_on = false;
     rocblas_handle blas = nullptr;
@@ -946,6 +947,7 @@ struct StagePlan {
         if (bsr_on && !bsr.uploaded) {   // once: the host copy of the nonzeros is released after it
             upload(bsr.d_tasks, bsr.tasks, st);
             upload(bsr.d_runs, bsr.runs, st);
+            upload(bsr.d_tile_cols, bsr.tile_cols, st);
             // the W tiles in the three arithmetics: FP64 zero-filled and the nonzeros scattered into
             // it; FP32 and the bf16 split of the FP32 value converted on the device
             const uint64_t nw = bsr.tiles * uint64_t(S_BSR_TILE_N) * S_BSR_TILE_K;
@@ -1017,7 +1019,7 @@ struct StagePlan {
                     const void* b0 = mode == MODE_F64 ? bsr.d_w64.p : mode == MODE_F32 ? bsr.d_w32.p : bsr.d_whi.p;
                     const void* b1 = mode == MODE_BF16X3 ? bsr.d_wlo.p : nullptr;
                     HIPCHK(launch_s_bsr(st, mode, bsr.d_tasks.as<BsrTask>(), uint32_t(bsr.tasks.size()),
-                                        bsr.d_runs.as<BsrRun>(), b0, b1, b.p[BASE_WS], bsr.narrow));
+                                        bsr.d_runs.as<BsrRun>(), bsr.d_tile_cols.as<uint32_t>(), b0, b1, b.p[BASE_WS], bsr.narrow));
                 }
                 run_lib(st, b, mode);
                 if (!mixed) run_gather(st, b.p[BASE_WS], b.p[BASE_WS]);
@@ -2088,6 +2090,7 @@ void add_bsr_groups(StagePlan::Bsr& B, const std::vector<GroupedLowering::Group>
     std::vector<uint64_t> e0(ng + 1, 0);
     for (size_t gi = 0; gi < ng; ++gi) e0[gi + 1] = e0[gi] + (sc[gi].tiles ? wg[gi].size() : 0);
     B.n_ent = e0[ng];
+    B.tile_cols.assign(std::max<uint64_t>(tile0[ng], 1), 0u);
 #pragma omp parallel for schedule(dynamic, 1)
     for (int gi = 0; gi < int(ng); ++gi) {
         if (!sc[gi].tiles) continue;
@@ -2099,6 +2102,7 @@ void add_bsr_groups(StagePlan::Bsr& B, const std::vector<GroupedLowering::Group>
             const uint64_t tile = tile0[gi] + A[uint64_t(j) * nkt + t];
             B.ent_pos[q] = tile * (uint64_t(TN) * TK) + uint64_t(e.n - j * TN) * TK + (e.k - t * TK);
             B.ent_val[q] = e.v;
+            B.tile_cols[tile] |= 1u << ((e.n - j * TN) / 16);   // the group's tiles are this iteration's own
             ++q;
         }
     }
@@ -2141,6 +2145,12 @@ void add_bsr_groups(StagePlan::Bsr& B, const std::vector<GroupedLowering::Group>
                                            pr[j].second, 0u});
                     }
         B.flops += 2ull * g.M * S.visited;
+    }
+    if (g_trace) {
+        uint64_t on = 0;
+        for (uint32_t c : B.tile_cols) on += __builtin_popcount(c);
+        std::fprintf(stderr, "[mq] S tiles %llu, 16-column blocks with a nonzero %.3f\n", (unsigned long long)B.tiles + tile0[ng],
+                     tile0[ng] ? double(on) / (8.0 * double(tile0[ng])) : 0.0);
     }
     B.tiles = tile0[ng];
 }
@@ -3575,7 +3585,7 @@ int mq_plan_workspace_bytes(const mq_plan* p, uint64_t* bytes) {
     return guarded([&] {
         MQ_REQUIRE(p && bytes, "bad argument");
         const StagePlan& P = p->st;
-        *bytes = p->ws.bytes + p->ws32.bytes + p->part.bytes + P.gT.device_bytes() + P.gF.device_bytes() + P.bsr.d_tasks.bytes + P.bsr.d_runs.bytes + P.bsr.d_w64.bytes + P.bsr.d_w32.bytes + P.bsr.d_whi.bytes + P.bsr.d_wlo.bytes + P.red.device_bytes() + P.d_maps.bytes + P.d_units.bytes + P.d_rows.bytes + P.d_regions.bytes +
+        *bytes = p->ws.bytes + p->ws32.bytes + p->part.bytes + P.gT.device_bytes() + P.gF.device_bytes() + P.bsr.d_tasks.bytes + P.bsr.d_runs.bytes + P.bsr.d_tile_cols.bytes + P.bsr.d_w64.bytes + P.bsr.d_w32.bytes + P.bsr.d_whi.bytes + P.bsr.d_wlo.bytes + P.red.device_bytes() + P.d_maps.bytes + P.d_units.bytes + P.d_rows.bytes + P.d_regions.bytes +
                  P.d_small.bytes + P.d_src_off.bytes + P.d_alpha.bytes;
     });
 }

@@ -170,8 +170,9 @@ struct BsrRun {
 // bf16 hi / lo tiles
 // narrow: every task's T_D step window, (32 * ld + S_BSR_TILE_M) elements of 8 bytes, fits in 2^32
 // bytes, so the kernel addresses it with 32-bit offsets from a uniform base
+// tile_cols: per W tile, bit j set if its columns 16 j .. 16 j + 15 hold a nonzero
 hipError_t launch_s_bsr(hipStream_t st, int mode, const BsrTask* tasks, uint32_t n_tasks, const BsrRun* runs,
-                        const void* bt0, const void* bt1, void* ws, bool narrow);
+                        const uint32_t* tile_cols, const void* bt0, const void* bt1, void* ws, bool narrow);
 
 // Side tables of a launch: remap entries, column units, row units, block scales.
 struct GemmTables {

@@ -1,0 +1,61 @@
+"""The T, S and final stage kernels at the shapes where a tile or a pipeline can go wrong: sectors
+smaller and larger than a tile, odd sizes, chain ends, groups of one and of few key tiles, against
+the CPU oracle."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as O
+from mqdmrg import engine as E
+from mqdmrg.workloads import SyntheticSite
+
+pytestmark = pytest.mark.gpu
+
+# FP64: sums of ~1e3 terms of either sign, each rounded to 2^-53.  FP32: each product and partial sum
+# rounded to 2^-24.  BF16x3: operands kept to 2^-17 (x = hi + lo).  Errors of different terms add
+# like random signs, so the norm of the difference stays near the rounding of one term; the
+# factors below are ~100 of it.
+RTOL = {E.PREC_F64: 1e-13, E.PREC_F32: 1e-5, E.PREC_BF16X3: 1e-3}
+
+SHAPES = [
+    ("heisenberg", 16, 7, 150),   # few keys (one or two key tiles), sectors of 1 to 60
+    ("heisenberg", 12, 1, 64),    # left end
+    ("hubbard", 12, 5, 301),
+    ("hubbard", 10, 7, 90),       # right end
+    ("qc", 8, 3, 77),
+    ("qc", 10, 1, 60),
+    ("qc_su2", 10, 4, 131),
+    ("qc_su2", 12, 8, 57),
+]
+
+
+@pytest.fixture(scope="module")
+def eng():
+    e = E.Engine(0)
+    yield e
+    e.close()
+
+
+@pytest.mark.parametrize("model,L,site,m", SHAPES)
+def test_sigma_stages_match_oracle(eng, model, L, site, m):
+    ws = SyntheticSite(model, L, site, m, seed=L + m)
+    Lc, Rc = ws.random_cohorts(ws.left_index), ws.random_cohorts(ws.right_index)
+    host = [O.HostBoundary(i, [x if x is not None else np.zeros(0) for x in c])
+            for i, c in ((ws.left_index, Lc), (ws.right_index, Rc))]
+    psi_h = ws.random_psi()
+    ref = O.SigmaOracle(ws.site_desc, ws.mpo_desc, *host).apply(psi_h)
+    Lb, Rb = E.DeviceBoundary.upload(eng, ws.left_index, Lc), E.DeviceBoundary.upload(eng, ws.right_index, Rc)
+    plan = E.SigmaPlan(eng, ws.site_desc, ws.mpo_desc, Lb, Rb)
+    psi = torch.from_numpy(psi_h).to("cuda:0")
+    for prec, tol in RTOL.items():
+        out = torch.full_like(psi, float("nan"))
+        plan.apply(psi, out, precision=prec)
+        eng.sync()
+        err = np.linalg.norm(out.cpu().numpy() - ref) / np.linalg.norm(ref)
+        print("%s L=%d site=%d m=%d precision %d: %.2e" % (model, L, site, m, prec, err), flush=True)
+        assert err <= tol
+        first = out.clone()
+        for _ in range(3):   # captured on the second application, replayed after it
+            plan.apply(psi, out, precision=prec)
+            eng.sync()
+            assert torch.equal(first, out)
