@@ -109,7 +109,7 @@ void f_unit_kernel(const GemmTask* __restrict__ tasks, uint32_t n_tasks, const G
     const GemmUnit* __restrict__ units = tables.units;
     const double* __restrict__ scales = tables.scales;
 
-    const uint32_t tile = xcd_tile(blockIdx.x, gridDim.x);
+    const uint32_t tile = xcd_tile_cyclic<16>(blockIdx.x, gridDim.x);
     const GemmTask tk = tasks[f_task_of(tasks, n_tasks, tile_task, tile)];
     const uint32_t M = tk.M, N = tk.N;
     const uint32_t local = tile - tk.tile_begin;

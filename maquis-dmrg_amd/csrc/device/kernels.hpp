@@ -132,6 +132,20 @@ __device__ inline uint32_t xcd_tile(uint32_t b, uint32_t n) {
     return x < r ? x * (q + 1) + i : r * (q + 1) + (x - r) * q + i;
 }
 
+// As xcd_tile, in chunks of C tiles dealt to the XCDs in turn.  Tiles differ in work (K runs, segment
+// lengths), and neighbours are alike: with one contiguous range per XCD some XCDs finished long before
+// others (CUs busy 80% of the FP64 S stage and 72% of the T stage at SU2U1 L=24 m=1000); a chunk still
+// shares its panels in one L2.  SU2U1 L=30 m=1500, contiguous ranges -> chunks: FP64 T stage (C = 32)
+// 22.8 -> 18.5 ms, S stage (C = 64, its 8 x 8 panel blocks) 38.4 -> 31.1, final stage (C = 16) 14.2 ->
+// 13.5; BF16x3 6.5 -> 5.5, 10.9 -> 9.3, 7.3 -> 7.2.
+template <uint32_t C> __device__ inline uint32_t xcd_tile_cyclic(uint32_t b, uint32_t n) {
+    constexpr uint32_t X = 8;
+    const uint32_t full = n / (X * C) * (X * C);
+    if (b >= full) return full + xcd_tile(b - full, n - full);
+    const uint32_t x = b % X, i = b / X;
+    return (i / C * X + x) * C + i % C;
+}
+
 constexpr uint32_t MAP_NONE = 0xffffffffu;
 // Arithmetic of an application (mq_precision).  MODE_BF16X3: split products (hi*lo + lo*hi + hi*hi
 // of bf16 hi / lo parts, FP32 accumulation) in the S-stage kernel and the lean 128 x 128 T and

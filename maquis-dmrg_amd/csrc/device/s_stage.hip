@@ -98,8 +98,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void s_
     constexpr bool BF = MODE == MODE_BF16X3;
     __shared__ __align__(16) BsrSmem<MODE> sm[2];
 
-    // consecutive tasks (blocks of 8 x 8 panels of one group) run next to each other on one XCD
-    const uint32_t tile = xcd_tile(blockIdx.x, gridDim.x);
+    // a block of 8 x 8 panels of one group (64 tasks) runs on one XCD; the blocks are dealt to the XCDs in turn
+    const uint32_t tile = xcd_tile_cyclic<64>(blockIdx.x, gridDim.x);
     const BsrTask tk = tasks[tile];
     const T* __restrict__ A = reinterpret_cast<const T*>(ws) + tk.a_off;
     T* __restrict__ C = reinterpret_cast<T*>(ws) + tk.c_off;

@@ -98,7 +98,7 @@ void t_stack_kernel(const GemmTask* __restrict__ tasks, uint32_t n_tasks, const 
     const uint32_t* __restrict__ maps = tables.maps;
     const GemmRow* __restrict__ rows = tables.rows;
 
-    const uint32_t tile = xcd_tile(blockIdx.x, gridDim.x);
+    const uint32_t tile = xcd_tile_cyclic<32>(blockIdx.x, gridDim.x);
     const GemmTask tk = tasks[task_of(tasks, n_tasks, tile_task, tile)];
     const GemmSeg sg = segs[tk.seg0];
     const uint32_t M = tk.M, N = tk.N, K = sg.K;
