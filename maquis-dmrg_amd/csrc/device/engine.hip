@@ -375,7 +375,27 @@ struct GemmStage {
     // per tile configuration (128x128 and 64x64): every task of it suits the lean stacked T-stage
     // kernel (t_stage.hip) / the lean column-unit final-stage kernel (f_stage.hip)
     bool stacked[GEMM_N_CFG] = {}, units[GEMM_N_CFG] = {};
+    // stacked tasks run by the streamed T kernel instead, per K class (stream_class)
+    struct Stream {
+        std::vector<GemmTask> tasks;
+        uint32_t tiles = 0, strip = 0;
+        std::vector<uint32_t> tile_task;
+        DevBuf d_tasks, d_tile_task;
+    } stream[T_STREAM_N];
+    std::vector<int8_t> cls_of;   // per task of `all`: its class, -1 for the tile configurations
 
+    // The class of a task that the streamed T kernel takes, -1 if it does not: its 4 waves of 32
+    // columns need 128 columns to be busy (T_D of the ab initio chains: hundreds to thousands; the
+    // spin and Hubbard chains' narrower tasks stay with the 64 x 64 tiles).  Tasks of at most 32 rows
+    // keep the generic kernel, whose summation order (and FP32 arithmetic in BF16x3) is its own.
+    static int stream_class(const GemmTask& t, const std::vector<GemmSeg>& segs) {
+        if (t.rowunit == MAP_NONE || t.seg1 != t.seg0 + 1 || t.beta || t.M <= 32 || t.N < 128) return -1;
+        const GemmSeg& g = segs[t.seg0];
+        if (g.amap != MAP_NONE || g.bmap != MAP_NONE || g.units != MAP_NONE || g.trans_a || !g.K) return -1;
+        for (int c = 0; c < T_STREAM_N; ++c)
+            if (g.K <= T_STREAM_KMAX[c]) return c;
+        return -1;
+    }
     // Flops per size class: the block-size histogram the autotuner's decisions are keyed on.
     std::vector<uint64_t> class_flops(const std::vector<GemmSeg>& segs) const {
         std::vector<uint64_t> f(N_SIZE_CLASS, 0);
@@ -383,13 +403,33 @@ struct GemmStage {
             for (uint32_t s = t.seg0; s < t.seg1; ++s) f[size_class(t.M)] += 2ull * t.M * t.N * segs[s].K;
         return f;
     }
-    void build(const std::vector<GemmTask>& tasks) {
+    // streamed: take the streamed T kernel for the tasks it suits (plans whose T stage writes T_D in its
+    // own type: all but the library S stage's)
+    void build(const std::vector<GemmTask>& tasks, const std::vector<GemmSeg>& segs, bool streamed = false) {
+        static const bool generic = std::getenv("MQ_T_GENERIC") != nullptr;
         all = tasks;
+        cls_of.assign(all.size(), -1);
+        if (streamed && !generic)
+            for (size_t i = 0; i < all.size(); ++i) cls_of[i] = int8_t(stream_class(all[i], segs));
         rebuild();
+    }
+    static std::vector<uint32_t> tiles_to_tasks(const std::vector<GemmTask>& ts, uint64_t total) {
+        std::vector<uint32_t> tt;
+        if (ts.size() <= 64 || total == ts.size() || total >= (1ull << 28)) return tt;
+        tt.reserve(total);
+        for (uint32_t i = 0; i < ts.size(); ++i)
+            tt.insert(tt.end(), (i + 1 < ts.size() ? ts[i + 1].tile_begin : uint32_t(total)) - ts[i].tile_begin, i);
+        return tt;
     }
     void rebuild() {
         for (auto& c : cfg) c.clear();
-        for (const auto& t : all) {
+        for (auto& s : stream) s.tasks.clear();
+        for (size_t i = 0; i < all.size(); ++i) {
+            const GemmTask& t = all[i];
+            if (cls_of[i] >= 0) {
+                stream[cls_of[i]].tasks.push_back(t);
+                continue;
+            }
             int c = policy.cls[size_class(t.M)];
             if (c < 0) c = gemm_pick_cfg(t.M, t.N);
             // the split-K 16x16 kernel covers one 16x16 tile; column units, row units and remapped
@@ -407,15 +447,24 @@ struct GemmStage {
                 MQ_REQUIRE(tile < (1ull << 31), "too many GEMM tiles in one launch");
             }
             tiles[c] = uint32_t(tile);
-            tile_task[c].clear();
-            if (cfg[c].size() > 64 && tile != cfg[c].size() && tile < (1ull << 28)) {
-                tile_task[c].reserve(tile);
-                for (uint32_t t = 0; t < cfg[c].size(); ++t) {
-                    const GemmTask& k = cfg[c][t];
-                    const uint64_t n = uint64_t((k.M + GEMM_CFG_BM[c] - 1) / GEMM_CFG_BM[c]) * k.tiles_n;
-                    tile_task[c].insert(tile_task[c].end(), n, t);
+            tile_task[c] = tiles_to_tasks(cfg[c], tile);
+        }
+        for (int c = 0; c < T_STREAM_N; ++c) {
+            Stream& s = stream[c];
+            // long strips stage A rarely, short ones give small stages enough workgroups: the longest
+            // that leaves 8 workgroups per CU
+            for (s.strip = 1024;; s.strip /= 2) {
+                uint64_t tile = 0;
+                for (auto& t : s.tasks) {
+                    t.tiles_n = (t.N + s.strip - 1) / s.strip;
+                    t.tile_begin = uint32_t(tile);
+                    tile += uint64_t((t.M + T_STREAM_ROWS[c] - 1) / T_STREAM_ROWS[c]) * t.tiles_n;
+                    MQ_REQUIRE(tile < (1ull << 31), "too many GEMM tiles in one launch");
                 }
+                s.tiles = uint32_t(tile);
+                if (tile >= 2048 || s.strip == 256) break;
             }
+            s.tile_task = tiles_to_tasks(s.tasks, s.tiles);
         }
     }
     void upload_all(const std::vector<GemmSeg>& segs, hipStream_t st) {
@@ -449,8 +498,21 @@ struct GemmStage {
             upload(d_tasks[c], cfg[c], st);
             upload(d_tile_task[c], tile_task[c], st);
         }
+        for (auto& s : stream) {
+            if (s.tasks.empty()) continue;
+            upload(s.d_tasks, s.tasks, st);
+            upload(s.d_tile_task, s.tile_task, st);
+        }
     }
     void run(hipStream_t st, int mode, const char* types, Bases b, GemmTables tb) const {
+        for (int c = 0; c < T_STREAM_N; ++c) {
+            const Stream& s = stream[c];
+            if (!s.tiles) continue;
+            MQ_REQUIRE(mode == MODE_F64 || std::strcmp(types, "ddf") == 0, "streamed T tasks write T_D in its own type");
+            HIPCHK(launch_t_stream(st, c, mode, mode != MODE_F64, s.d_tasks.as<GemmTask>(), uint32_t(s.tasks.size()),
+                                   d_segs.as<GemmSeg>(), s.tiles, s.strip, b, tb,
+                                   s.tile_task.empty() ? nullptr : s.d_tile_task.as<uint32_t>()));
+        }
         for (int c = 0; c < GEMM_N_CFG; ++c) {
             if (!tiles[c]) continue;
             const uint32_t* tt = tile_task[c].empty() ? nullptr : d_tile_task[c].as<uint32_t>();
@@ -473,6 +535,7 @@ struct GemmStage {
         uint64_t n = d_segs.bytes;
         for (const auto& d : d_tasks) n += d.bytes;
         for (const auto& d : d_tile_task) n += d.bytes;
+        for (const auto& s : stream) n += s.d_tasks.bytes + s.d_tile_task.bytes;
         return n;
     }
 };
@@ -724,9 +787,9 @@ struct StagePlan {
     uint64_t sizes[N_BASES] = {0, 0, 0, 0, 0, 0};   // element counts of each base for validation
 
     void finish_tables() {
-        gT.build(t_tasks);
-        gF.build(f_tasks);
-        gU.build(u_tasks);
+        gT.build(t_tasks, t_segs, bsr_on);
+        gF.build(f_tasks, f_segs);
+        gU.build(u_tasks, u_segs);
         red.finish();
         std::vector<GatherRegion> big;
         for (const auto& r : regions) {

@@ -209,6 +209,13 @@ hipError_t launch_gemm(hipStream_t st, int cfg, int mode, const char* types, con
 // same tables, tiles per task and results as launch_gemm with that cfg.
 hipError_t launch_t_stack(hipStream_t st, int cfg, int mode, bool c_float, const GemmTask* tasks, uint32_t n_tasks,
                           const GemmSeg* segs, uint32_t n_tiles, Bases bases, GemmTables tb, const uint32_t* tile_task);
+// The same tasks on the streamed kernel of t_stage.hip, in classes of K (K <= T_STREAM_KMAX[cls]):
+// tiles of T_STREAM_ROWS[cls] rows and `strip` columns, row tile fastest.
+constexpr int T_STREAM_N = 3;
+constexpr uint32_t T_STREAM_KMAX[T_STREAM_N] = {64, 144, 288}, T_STREAM_ROWS[T_STREAM_N] = {64, 64, 32};
+hipError_t launch_t_stream(hipStream_t st, int cls, int mode, bool c_float, const GemmTask* tasks, uint32_t n_tasks,
+                           const GemmSeg* segs, uint32_t n_tiles, uint32_t strip, Bases bases, GemmTables tb,
+                           const uint32_t* tile_task);
 // Final-stage tasks of tile configuration cfg (GEMM_CFG_128x128 or GEMM_CFG_64x64) whose segments
 // all read B through column units (no row units, no B block map, no beta, m_off 0) on the lean
 // kernel of f_stage.hip: MODE_F64 (all double), MODE_F32 or MODE_BF16X3 (A double, B float,

@@ -331,6 +331,331 @@ void t_stack_kernel(const GemmTask* __restrict__ tasks, uint32_t n_tasks, const 
     }
 }
 
+// The streamed form of the stacked tasks: a workgroup of NW waves keeps 16 RB rows of A in LDS for the
+// whole K range (K <= KP) and streams a strip of `strip` columns past them; each wave takes chunks of
+// WC = 16 CB columns.  A step's B (WC columns x 16 keys) goes from memory to the wave's own part of LDS
+// ([n][k], the next step's loads in flight meanwhile) and from there into the MFMA lane layout, so no
+// barrier follows the staging of A and the waves drift freely: stores of one overlap products of
+// another.
+//
+// What bounds it: the stores of T_D (in segments of one sector's rows), in FP64 the matrix cores
+// beside them.  T's products are short (K is one sector: 75 keys by flops at SU2U1 L=24 m=1000) and its
+// output large, so tiles of 128 x 128 spent most of their time filling and draining, in FP64 at one
+// wave per SIMD.  Here A is read, scaled, converted and (BF16X3) split once per strip instead of once
+// per column tile, and every B element is read and converted by one wave.  Neighbouring lanes always
+// touch neighbouring addresses, which the vector cache's rate of one line per cycle asks for: B by
+// runs of 16 keys, and T_D along its rows, with the MFMA operands exchanged (D = B^T A^T: lane l16 is
+// a row of A, the four accumulators are columns).  T stage in ms, t_stack_kernel -> this: SU2U1 L=30
+// m=1500 FP64 18.5 -> 10.1, BF16X3 5.5 -> 5.1; L=24 m=1000 4.4 -> 2.3 and 1.40 -> 1.30; L=16 m=256
+// BF16X3 0.061 -> 0.051.  (B straight from memory in the MFMA layout, whose neighbouring lanes are
+// different columns: FP64 11.0, BF16X3 5.9 at L=30; stores along the columns: slower still.)
+//
+// Classes by K: 64 rows of A up to K = 64 take 34 KB in FP64, three workgroups of 4 waves per CU;
+// up to 144 75 KB, one workgroup of 8 waves; up to 288 32 rows fit beside the 8 waves' buffers.
+//
+// Same products, key slots and step order as t_stack_kernel: bitwise the same T_D.
+// LDS accesses of one wave execute in program order; this keeps the compiler from moving them
+__device__ inline void wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+template <int MODE> constexpr int TP_PAD = MODE == MODE_F64 ? 2 : MODE == MODE_F32 ? 4 : 8;   // odd number of 16-byte runs per row
+
+template <int MODE, typename TC, int KP, int RB, int NW>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(MODE == MODE_BF16X3 ? 4 : MODE == MODE_F64 && NW == 8 ? 2 : 3)))
+void t_stream_kernel(const GemmTask* __restrict__ tasks, uint32_t n_tasks, const GemmSeg* __restrict__ segs,
+                     Bases bases, GemmTables tables, const uint32_t* __restrict__ tile_task, uint32_t strip) {
+    typedef typename TsTraits<MODE>::T T;
+    typedef typename TsTraits<MODE>::Acc Acc;
+    constexpr bool BF = MODE == MODE_BF16X3;
+    constexpr int CB = 2, TM = 16 * RB, WC = 16 * CB, KPT = TK * TM / (64 * NW);
+    constexpr int P = KP + TP_PAD<MODE>, PB = TK + TP_PAD<MODE>;
+    static_assert(KPT >= 1 && KP % TK == 0, "A staging");
+    typedef typename std::conditional<BF, uint16_t, T>::type E;
+    __shared__ __align__(16) E sa[BF ? 2 : 1][TM][P];          // BF16X3: hi, lo
+    struct Wave {   // one wave's own: a step of B, or (between chunks) the C offsets of a chunk's columns
+        union {
+            E b[BF ? 2 : 1][WC][PB];
+            uint64_t off[RB][WC];
+        };
+    };
+    __shared__ __align__(16) Wave sw[NW];
+    const uint32_t* __restrict__ maps = tables.maps;
+    const GemmRow* __restrict__ rows = tables.rows;
+
+    const uint32_t tile = xcd_tile_cyclic<8>(blockIdx.x, gridDim.x);
+    const GemmTask tk = tasks[task_of(tasks, n_tasks, tile_task, tile)];
+    const GemmSeg sg = segs[tk.seg0];
+    const uint32_t M = tk.M, N = tk.N, K = sg.K;
+    const uint32_t local = tile - tk.tile_begin, tiles_m = (M + TM - 1) / TM;
+    const uint32_t m0 = (local % tiles_m) * TM, n_begin = (local / tiles_m) * strip, n_end = min(N, n_begin + strip);
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int l16 = lane & 15, lk = lane >> 4;
+    const uint32_t steps = (K + TK - 1) / TK;
+
+    // ---- A: thread t stages row t % TM, keys (t / TM) KPT .. of every step (keys beyond K as zero)
+    {
+        const int am = tid % TM, ak = (tid / TM) * KPT;
+        const uint32_t m = min(m0 + uint32_t(am), M - 1);
+        const GemmRow R = rows[maps[tk.rowunit + m / 16]];
+        const uint32_t i = min(m - R.row0, R.nrows - 1);
+        const double* __restrict__ a_row = bases.p[sg.a_base] + sg.a_off + R.a_src + uint64_t(i) * R.a_si;
+        const T a_sc = T(R.a_scale * sg.alpha);
+#pragma unroll 2
+        for (uint32_t s = 0; s < steps; ++s) {
+            T x[KPT];
+#pragma unroll
+            for (int e = 0; e < KPT; ++e) {
+                const uint32_t k = s * TK + ak + e;
+                x[e] = T(a_row[uint64_t(min(k, K - 1)) * R.a_sk]) * a_sc;
+                if (k >= K) x[e] = T(0);
+            }
+            E* d = &sa[0][am][s * TK + ak];
+#pragma unroll
+            for (int e = 0; e < KPT; ++e) {
+                if constexpr (BF) {
+                    uint32_t h, l;
+                    split2(x[e], 0.f, h, l);
+                    d[e] = uint16_t(h);
+                    d[TM * P + e] = uint16_t(l);
+                } else {
+                    d[e] = x[e];
+                }
+            }
+        }
+    }
+    __syncthreads();
+
+    const double* __restrict__ B = bases.p[sg.b_base] + sg.b_off;
+    TC* __restrict__ C = reinterpret_cast<TC*>(bases.p[tk.c_base]) + tk.c_off;
+    const uint32_t cbw = max(tk.cbw, 1u);
+    E(*wb)[WC][PB] = sw[wave].b;
+
+    // ---- where T_D's elements go.  The lane's row of every 16-row block: its offset in the block's unit,
+    // ~0 if it is padding.
+    uint32_t rowoff[RB];
+#pragma unroll
+    for (int i = 0; i < RB; ++i) {
+        const uint32_t mb = min(m0 + 16 * i, M - 16);
+        const GemmRow& R = rows[maps[tk.rowunit + mb / 16]];
+        const uint32_t li = mb + l16 - R.row0;
+        rowoff[i] = m0 + 16 * i < M && li < R.nrows ? li * R.c_si : ~0u;
+    }
+    // The units whose column offsets the lane computes: column lane % 32 of a chunk, row blocks
+    // lane / 32 + 2 p (a chunk's offsets go through LDS; their map entries are loaded at its start)
+    static_assert(WC == 32 && RB % 2 == 0, "two row blocks per pass");
+    constexpr int NP = RB / 2;
+    uint64_t u_src[NP];
+    uint32_t u_cmap[NP], u_cldk[NP], u_ldc[NP];
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+        const GemmRow& R = rows[maps[tk.rowunit + min(m0 + 16 * (lane / 32 + 2 * p), M - 16) / 16]];
+        u_src[p] = R.c_src;
+        u_cmap[p] = R.cmap;
+        u_cldk[p] = R.cldk;
+        u_ldc[p] = R.ldc;
+    }
+
+    auto body = [&](auto trans) {
+        constexpr bool TB = decltype(trans)::value;
+        const uint64_t ldb = sg.ldb;
+        // B of a step, NV pairs of doubles per lane: stored cohort (k contiguous): pair v is keys
+        // 2 (lane % 8) of column lane / 8 + 8 v; transposed (n contiguous): columns 2 (lane % (WC / 2)),
+        // key lane / (WC / 2) + (128 / WC) v
+        constexpr int NV = WC / 8;
+        d2_a8 vb[NV];
+        const int b_n = TB ? 2 * (lane % (WC / 2)) : lane / 8, b_k = TB ? lane / (WC / 2) : 2 * (lane % 8);
+        auto load = [&](uint32_t c, uint32_t s) {   // keys beyond K and columns beyond N read the last one
+#pragma unroll
+            for (int v = 0; v < NV; ++v) {
+                if constexpr (TB) {
+                    const uint32_t n = c + b_n;
+                    const double* p = B + uint64_t(min(s * TK + b_k + (128 / WC) * v, K - 1)) * ldb;
+                    vb[v][0] = p[min(n, N - 1)];
+                    vb[v][1] = p[min(n + 1, N - 1)];
+                } else {
+                    const double* p = B + uint64_t(min(c + b_n + 8 * v, N - 1)) * ldb;
+                    const uint32_t k = s * TK + b_k;
+                    if ((s + 1) * TK <= K) {
+                        vb[v] = *reinterpret_cast<const d2_a8*>(p + k);
+                    } else {
+                        vb[v][0] = p[min(k, K - 1)];
+                        vb[v][1] = p[min(k + 1, K - 1)];
+                    }
+                }
+            }
+        };
+        // BF16X3: bf16 hi / lo of two elements of B.  t_stack_kernel's compiled form rounds the first step's
+        // hi from the FP64 value and the others' from its FP32 rounding; so does this.  They differ only
+        // where the FP32 value lies halfway between two bf16 (tie), so the longer conversion runs only
+        // for a first step that holds one (one in a hundred).
+        auto split = [&](double dx, double dy, auto first, uint32_t& h, uint32_t& l) {
+            const float x = float(dx), y = float(dy);
+            if constexpr (decltype(first)::value)
+                h = __builtin_bit_cast(uint32_t, bf2{(__bf16)dx, (__bf16)dy});
+            else   // (a C++ conversion of x would be folded into one of dx)
+                asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(h) : "v"(x), "v"(y));
+            l = __builtin_bit_cast(uint32_t, bf2{(__bf16)(x - __uint_as_float(h << 16)),
+                                                 (__bf16)(y - __uint_as_float(h & 0xffff0000u))});
+        };
+        auto put = [&](auto first) {   // the loaded step into the wave's LDS, in the arithmetic's type
+#pragma unroll
+            for (int v = 0; v < NV; ++v) {
+                const T x = T(vb[v][0]), y = T(vb[v][1]);
+                if constexpr (TB) {
+                    const int k = b_k + (128 / WC) * v;
+                    if constexpr (BF) {
+                        uint32_t h, l;
+                        split(vb[v][0], vb[v][1], first, h, l);
+                        wb[0][b_n][k] = uint16_t(h);
+                        wb[0][b_n + 1][k] = uint16_t(h >> 16);
+                        wb[1][b_n][k] = uint16_t(l);
+                        wb[1][b_n + 1][k] = uint16_t(l >> 16);
+                    } else {
+                        wb[0][b_n][k] = x;
+                        wb[0][b_n + 1][k] = y;
+                    }
+                } else {
+                    const int n = b_n + 8 * v;
+                    if constexpr (BF) {
+                        uint32_t h, l;
+                        split(vb[v][0], vb[v][1], first, h, l);
+                        *reinterpret_cast<uint32_t*>(&wb[0][n][b_k]) = h;
+                        *reinterpret_cast<uint32_t*>(&wb[1][n][b_k]) = l;
+                    } else {
+                        typedef T t2 __attribute__((ext_vector_type(2)));
+                        *reinterpret_cast<t2*>(&wb[0][n][b_k]) = t2{x, y};
+                    }
+                }
+            }
+        };
+        uint32_t c = n_begin + wave * WC;
+        if (c >= n_end) return;
+        load(c, 0);
+        while (true) {
+            Acc acc[RB][CB];
+#pragma unroll
+            for (int i = 0; i < RB; ++i)
+#pragma unroll
+                for (int j = 0; j < CB; ++j) acc[i][j] = Acc{0, 0, 0, 0};
+            const uint32_t oc = min(c + lane % 32, n_end - 1), oblk = oc / cbw, oin = oc - oblk * cbw;
+            uint32_t om[NP];
+#pragma unroll
+            for (int p = 0; p < NP; ++p) om[p] = u_cmap[p] != MAP_NONE ? maps[u_cmap[p] + oblk] : 0u;
+            const uint32_t next = c + NW * WC;
+            for (uint32_t s = 0; s < steps; ++s) {
+                bool halfway = false;
+                if (BF && s == 0) {
+#pragma unroll
+                    for (int v = 0; v < NV; ++v)
+#pragma unroll
+                        for (int e = 0; e < 2; ++e)
+                            halfway = halfway || (__float_as_uint(float(vb[v][e])) & 0xffffu) == 0x8000u;
+                    halfway = __any(halfway);
+                }
+                if (halfway) put(std::true_type{});
+                else put(std::false_type{});
+                // the next step's loads (or the next chunk's first; past the strip the last again)
+                const bool last = s + 1 == steps;
+                load(last ? min(next, n_end - 1) : c, last ? 0 : s + 1);
+                wave_fence();   // the wave's LDS accesses stay in this order
+                if constexpr (BF) {
+                    s4 bh[CB], bl[CB];
+#pragma unroll
+                    for (int j = 0; j < CB; ++j) {
+                        bh[j] = *reinterpret_cast<const s4*>(&wb[0][16 * j + l16][4 * lk]);
+                        bl[j] = *reinterpret_cast<const s4*>(&wb[1][16 * j + l16][4 * lk]);
+                    }
+#pragma unroll
+                    for (int i = 0; i < RB; ++i) {
+                        const s4 ah = *reinterpret_cast<const s4*>(&sa[0][16 * i + l16][s * TK + 4 * lk]);
+                        const s4 al = *reinterpret_cast<const s4*>(&sa[1][16 * i + l16][s * TK + 4 * lk]);
+#pragma unroll
+                        for (int j = 0; j < CB; ++j) {
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(bl[j], ah, acc[i][j], 0, 0, 0);
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(bh[j], al, acc[i][j], 0, 0, 0);
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(bh[j], ah, acc[i][j], 0, 0, 0);
+                        }
+                    }
+                } else {
+                    typedef T tv __attribute__((ext_vector_type(16 / sizeof(T))));
+                    constexpr int VN = 16 / sizeof(T);
+                    T a[RB][4], bb[CB][4];
+#pragma unroll
+                    for (int h = 0; h < 4 / VN; ++h) {
+#pragma unroll
+                        for (int j = 0; j < CB; ++j) {
+                            const tv x = *reinterpret_cast<const tv*>(&wb[0][16 * j + l16][4 * lk + VN * h]);
+#pragma unroll
+                            for (int e = 0; e < VN; ++e) bb[j][VN * h + e] = x[e];
+                        }
+#pragma unroll
+                        for (int i = 0; i < RB; ++i) {
+                            const tv x = *reinterpret_cast<const tv*>(&sa[0][16 * i + l16][s * TK + 4 * lk + VN * h]);
+#pragma unroll
+                            for (int e = 0; e < VN; ++e) a[i][VN * h + e] = x[e];
+                        }
+                    }
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+#pragma unroll
+                        for (int i = 0; i < RB; ++i)
+#pragma unroll
+                            for (int j = 0; j < CB; ++j) {
+                                if constexpr (MODE == MODE_F64)
+                                    acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(bb[j][e], a[i][e], acc[i][j], 0, 0, 0);
+                                else
+                                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bb[j][e], a[i][e], acc[i][j], 0, 0, 0);
+                            }
+                }
+                wave_fence();
+            }
+            // ---- store the chunk
+#pragma unroll
+            for (int p = 0; p < NP; ++p)
+                sw[wave].off[lane / 32 + 2 * p][lane % 32] =
+                    u_src[p] + (u_cmap[p] != MAP_NONE ? uint64_t(om[p]) * u_cldk[p] + uint64_t(oin) * u_ldc[p]
+                                                      : uint64_t(oc) * u_ldc[p]);
+            wave_fence();
+            // D = B^T A^T: lane l16 is row l16 of every 16-row block, accumulator r of block j the column
+            // 16 j + 4 r + lk (FP64) or 16 j + 4 lk + r
+#pragma unroll
+            for (int j = 0; j < CB; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int n = 16 * j + (MODE == MODE_F64 ? 4 * r + lk : 4 * lk + r);
+                    if (c + n >= n_end) continue;
+#pragma unroll
+                    for (int i = 0; i < RB; ++i)
+                        if (rowoff[i] != ~0u) C[sw[wave].off[i][n] + rowoff[i]] = TC(acc[i][j][r]);
+                }
+            wave_fence();
+            c = next;
+            if (c >= n_end) break;
+        }
+    };
+    if (sg.trans_b) body(std::true_type{});
+    else body(std::false_type{});
+}
+
+template <int MODE, typename TC>
+hipError_t launch_t_stream_mode(hipStream_t st, int cls, const GemmTask* tasks, uint32_t n_tasks, const GemmSeg* segs,
+                                uint32_t n_tiles, uint32_t strip, Bases bases, GemmTables tb,
+                                const uint32_t* tile_task) {
+#define MQ_T_STREAM(KP_, RB_, NW_)                                                                              \
+    hipLaunchKernelGGL((t_stream_kernel<MODE, TC, KP_, RB_, NW_>), dim3(n_tiles), dim3(64 * NW_), 0, st, tasks, \
+                       n_tasks, segs, bases, tb, tile_task, strip)
+    switch (cls) {
+        case 0: MQ_T_STREAM(T_STREAM_KMAX[0], T_STREAM_ROWS[0] / 16, 4); break;
+        case 1: MQ_T_STREAM(T_STREAM_KMAX[1], T_STREAM_ROWS[1] / 16, 8); break;
+        case 2: MQ_T_STREAM(T_STREAM_KMAX[2], T_STREAM_ROWS[2] / 16, 8); break;
+        default: return hipErrorInvalidValue;
+    }
+#undef MQ_T_STREAM
+    return hipGetLastError();
+}
+
 template <int BM>
 hipError_t launch_t_tile(hipStream_t st, int mode, bool c_float, const GemmTask* tasks, uint32_t n_tasks,
                          const GemmSeg* segs, uint32_t n_tiles, Bases bases, GemmTables tb, const uint32_t* tile_task) {
@@ -349,6 +674,19 @@ hipError_t launch_t_tile(hipStream_t st, int mode, bool c_float, const GemmTask*
 }
 
 }  // namespace
+
+hipError_t launch_t_stream(hipStream_t st, int cls, int mode, bool c_float, const GemmTask* tasks, uint32_t n_tasks,
+                           const GemmSeg* segs, uint32_t n_tiles, uint32_t strip, Bases bases, GemmTables tb,
+                           const uint32_t* tile_task) {
+    if (n_tiles == 0) return hipSuccess;
+    if (mode == MODE_F64 && !c_float)
+        return launch_t_stream_mode<MODE_F64, double>(st, cls, tasks, n_tasks, segs, n_tiles, strip, bases, tb, tile_task);
+    if (mode == MODE_F32 && c_float)
+        return launch_t_stream_mode<MODE_F32, float>(st, cls, tasks, n_tasks, segs, n_tiles, strip, bases, tb, tile_task);
+    if (mode == MODE_BF16X3 && c_float)
+        return launch_t_stream_mode<MODE_BF16X3, float>(st, cls, tasks, n_tasks, segs, n_tiles, strip, bases, tb, tile_task);
+    return hipErrorInvalidValue;
+}
 
 hipError_t launch_t_stack(hipStream_t st, int cfg, int mode, bool c_float, const GemmTask* tasks, uint32_t n_tasks,
                           const GemmSeg* segs, uint32_t n_tiles, Bases bases, GemmTables tb, const uint32_t* tile_task) {
