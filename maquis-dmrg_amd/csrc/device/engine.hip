@@ -364,6 +364,16 @@ struct TilePolicy {
     int cls[N_SIZE_CLASS] = {-1, -1, -1, -1, -1};
 };
 
+// Task of every tile of a launch of many multi-tile tasks (empty: the kernels search the task table).
+static std::vector<uint32_t> tiles_to_tasks(const std::vector<GemmTask>& ts, uint64_t total) {
+    std::vector<uint32_t> tt;
+    if (ts.size() <= 64 || total == ts.size() || total >= (1ull << 28)) return tt;
+    tt.reserve(total);
+    for (uint32_t i = 0; i < ts.size(); ++i)
+        tt.insert(tt.end(), (i + 1 < ts.size() ? ts[i + 1].tile_begin : uint32_t(total)) - ts[i].tile_begin, i);
+    return tt;
+}
+
 struct GemmStage {
     std::vector<GemmTask> all;                     // the lowering's tasks (rebuilt per policy)
     TilePolicy policy;
@@ -378,11 +388,47 @@ struct GemmStage {
     // stacked tasks run by the streamed T kernel instead, per K class (stream_class)
     struct Stream {
         std::vector<GemmTask> tasks;
-        uint32_t tiles = 0, strip = 0;
+        uint32_t tiles = 0, strip = 0, rows = 0;
         std::vector<uint32_t> tile_task;
         DevBuf d_tasks, d_tile_task;
+        void number(uint32_t rows, uint32_t cols) {
+            uint64_t tile = 0;
+            for (auto& t : tasks) {
+                t.tiles_n = (t.N + cols - 1) / cols;
+                t.tile_begin = uint32_t(tile);
+                tile += uint64_t((t.M + rows - 1) / rows) * t.tiles_n;
+                MQ_REQUIRE(tile < (1ull << 31), "too many GEMM tiles in one launch");
+            }
+            tiles = uint32_t(tile);
+        }
+        void finish() { tile_task = tiles_to_tasks(tasks, tiles); }
+        void upload_all(hipStream_t st) {
+            if (tasks.empty()) return;
+            upload(d_tasks, tasks, st);
+            upload(d_tile_task, tile_task, st);
+        }
+        const uint32_t* table() const { return tile_task.empty() ? nullptr : d_tile_task.as<uint32_t>(); }
+        uint64_t device_bytes() const { return d_tasks.bytes + d_tile_task.bytes; }
     } stream[T_STREAM_N];
     std::vector<int8_t> cls_of;   // per task of `all`: its class, -1 for the tile configurations
+    // column-unit tasks run by the wave form of the final stage, numbered for FP64 and for FP32: those
+    // of at most 32 rows, in FP64 every task of a small stage (wave64_all)
+    static constexpr int8_t WAVE = 100;
+    Stream wave64, wave32;
+    bool wave64_all = false, wave_tr = false;
+
+    static bool wave_task(const GemmTask& t, const std::vector<GemmSeg>& segs) {
+        if (t.rowunit != MAP_NONE || t.colunit == MAP_NONE || t.beta || t.m_off || t.cmap != MAP_NONE || !t.M || !t.N ||
+            t.seg1 <= t.seg0)
+            return false;
+        for (uint32_t k = t.seg0; k < t.seg1; ++k) {
+            const GemmSeg& g = segs[k];
+            if (g.units == MAP_NONE || g.bmap != MAP_NONE || g.trans_b || !g.K || g.K >= 65536 || !g.bbh || g.bbh >= 65536)
+                return false;
+            if (g.amap == MAP_NONE ? g.trans_a : (!g.trans_a || g.ascale == MAP_NONE)) return false;
+        }
+        return true;
+    }
 
     // The class of a task that the streamed T kernel takes, -1 if it does not: its 4 waves of 32
     // columns need 128 columns to be busy (T_D of the ab initio chains: hundreds to thousands; the
@@ -411,21 +457,37 @@ struct GemmStage {
         cls_of.assign(all.size(), -1);
         if (streamed && !generic)
             for (size_t i = 0; i < all.size(); ++i) cls_of[i] = int8_t(stream_class(all[i], segs));
+        static const bool generic_f = std::getenv("MQ_F_GENERIC") != nullptr;
+        if (!generic_f) {
+            // FP64: a stage whose 64 x 64 tiles would leave CUs idle runs in the wave form altogether
+            // (its chains split over 4 waves)
+            bool every = !all.empty();
+            uint64_t tiles64 = 0;
+            for (size_t i = 0; i < all.size(); ++i) {
+                const bool ok = wave_task(all[i], segs);
+                every = every && ok;
+                if (ok && all[i].M <= 32) cls_of[i] = WAVE;
+                if (all[i].M > 32) tiles64 += uint64_t((all[i].M + 63) / 64) * ((all[i].N + 63) / 64);
+            }
+            wave64_all = every && tiles64 < 256;
+            wave_tr = false;
+            for (const auto& g : segs) wave_tr = wave_tr || g.amap != MAP_NONE;
+        }
         rebuild();
-    }
-    static std::vector<uint32_t> tiles_to_tasks(const std::vector<GemmTask>& ts, uint64_t total) {
-        std::vector<uint32_t> tt;
-        if (ts.size() <= 64 || total == ts.size() || total >= (1ull << 28)) return tt;
-        tt.reserve(total);
-        for (uint32_t i = 0; i < ts.size(); ++i)
-            tt.insert(tt.end(), (i + 1 < ts.size() ? ts[i + 1].tile_begin : uint32_t(total)) - ts[i].tile_begin, i);
-        return tt;
     }
     void rebuild() {
         for (auto& c : cfg) c.clear();
         for (auto& s : stream) s.tasks.clear();
+        wave64.tasks.clear();
+        wave32.tasks.clear();
         for (size_t i = 0; i < all.size(); ++i) {
             const GemmTask& t = all[i];
+            if (cls_of[i] == WAVE) {
+                wave64.tasks.push_back(t);
+                wave32.tasks.push_back(t);
+                continue;
+            }
+            if (wave64_all) wave64.tasks.push_back(t);   // FP32 and BF16x3 keep their tiles
             if (cls_of[i] >= 0) {
                 stream[cls_of[i]].tasks.push_back(t);
                 continue;
@@ -454,17 +516,18 @@ struct GemmStage {
             // long strips stage A rarely, short ones give small stages enough workgroups: the longest
             // that leaves 8 workgroups per CU
             for (s.strip = 1024;; s.strip /= 2) {
-                uint64_t tile = 0;
-                for (auto& t : s.tasks) {
-                    t.tiles_n = (t.N + s.strip - 1) / s.strip;
-                    t.tile_begin = uint32_t(tile);
-                    tile += uint64_t((t.M + T_STREAM_ROWS[c] - 1) / T_STREAM_ROWS[c]) * t.tiles_n;
-                    MQ_REQUIRE(tile < (1ull << 31), "too many GEMM tiles in one launch");
-                }
-                s.tiles = uint32_t(tile);
-                if (tile >= 2048 || s.strip == 256) break;
+                s.number(T_STREAM_ROWS[c], s.strip);
+                if (s.tiles >= 2048 || s.strip == 256) break;
             }
-            s.tile_task = tiles_to_tasks(s.tasks, s.tiles);
+            s.finish();
+        }
+        for (Stream* w : {&wave64, &wave32}) {
+            // 32 rows per wave where that leaves 4 workgroups per CU, else 16
+            for (w->rows = 32;; w->rows = 16) {
+                w->number(w->rows, w == &wave64 ? F_WAVE_COLS_F64 : F_WAVE_COLS_F32);
+                if (w->tiles >= 1024 || w->rows == 16) break;
+            }
+            w->finish();
         }
     }
     void upload_all(const std::vector<GemmSeg>& segs, hipStream_t st) {
@@ -498,11 +561,9 @@ struct GemmStage {
             upload(d_tasks[c], cfg[c], st);
             upload(d_tile_task[c], tile_task[c], st);
         }
-        for (auto& s : stream) {
-            if (s.tasks.empty()) continue;
-            upload(s.d_tasks, s.tasks, st);
-            upload(s.d_tile_task, s.tile_task, st);
-        }
+        for (auto& s : stream) s.upload_all(st);
+        wave64.upload_all(st);
+        wave32.upload_all(st);
     }
     void run(hipStream_t st, int mode, const char* types, Bases b, GemmTables tb) const {
         for (int c = 0; c < T_STREAM_N; ++c) {
@@ -511,8 +572,15 @@ struct GemmStage {
             MQ_REQUIRE(mode == MODE_F64 || std::strcmp(types, "ddf") == 0, "streamed T tasks write T_D in its own type");
             HIPCHK(launch_t_stream(st, c, mode, mode != MODE_F64, s.d_tasks.as<GemmTask>(), uint32_t(s.tasks.size()),
                                    d_segs.as<GemmSeg>(), s.tiles, s.strip, b, tb,
-                                   s.tile_task.empty() ? nullptr : s.d_tile_task.as<uint32_t>()));
+                                   s.table()));
         }
+        const Stream& w = mode == MODE_F64 ? wave64 : wave32;
+        if (w.tiles) {   // (BF16x3 runs its tasks of at most 32 rows in FP32, as the generic kernel did)
+            MQ_REQUIRE(mode == MODE_F64 || std::strcmp(types, "dfd") == 0, "wave final-stage tasks read FP32 S_D");
+            HIPCHK(launch_f_wave(st, mode == MODE_F64 ? MODE_F64 : MODE_F32, int(w.rows / 16), wave_tr, w.d_tasks.as<GemmTask>(),
+                                 uint32_t(w.tasks.size()), d_segs.as<GemmSeg>(), w.tiles, b, tb, w.table()));
+        }
+        if (mode == MODE_F64 && wave64_all) return;
         for (int c = 0; c < GEMM_N_CFG; ++c) {
             if (!tiles[c]) continue;
             const uint32_t* tt = tile_task[c].empty() ? nullptr : d_tile_task[c].as<uint32_t>();
@@ -535,7 +603,8 @@ struct GemmStage {
         uint64_t n = d_segs.bytes;
         for (const auto& d : d_tasks) n += d.bytes;
         for (const auto& d : d_tile_task) n += d.bytes;
-        for (const auto& s : stream) n += s.d_tasks.bytes + s.d_tile_task.bytes;
+        for (const auto& s : stream) n += s.device_bytes();
+        n += wave64.device_bytes() + wave32.device_bytes();
         return n;
     }
 };

@@ -95,6 +95,12 @@ template <int N> __device__ inline void loadn(const float* p, float* v) {
     }
 }
 
+// LDS accesses of one wave execute in program order; this keeps the compiler from moving them
+__device__ inline void wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // BM x BM tiles, 2 x 2 waves of WB x WB 16 x 16 blocks
 template <int MODE, typename TB, int BM>
 __global__ __launch_bounds__(FT) __attribute__((amdgpu_waves_per_eu(BM == 64 ? 4 : 2)))
@@ -342,6 +348,258 @@ void f_unit_kernel(const GemmTask* __restrict__ tasks, uint32_t n_tasks, const G
     }
 }
 
+// The wave form of the final-stage tasks: one wave computes 16 RB rows x 16 columns of a task's block
+// over its whole K chain (FP32: the summation order is fixed), or the 4 waves of a workgroup take a
+// quarter of the chain each and add up through LDS in wave order (FP64, WK = 4).  For tasks of at most
+// 32 rows, and in FP64 for stages too small to fill the card with 64 x 64 tiles.
+//
+// What bounds it: latency.  Such a stage has few blocks and long chains (K of about 2048 per task, in
+// left cohorts of a dozen 16-key steps each): at SU2U1 L=16 m=256 its 137 tiles of the generic kernel
+// took 2.6 us per step, a map lookup, the loads behind it, a barrier.  Here every wave is its own
+// pipeline without barriers: the S_D columns (map entries) of a step are looked up one step before its
+// loads are issued, FD steps are loaded ahead, and the next segment's column unit is fetched while
+// the current one runs.  Lane l loads S_D column l / 4, keys 4 (l % 4) .. + 3 of the step (runs of one
+// column next to each other), turned into the MFMA layout in the wave's own LDS; A is read in that
+// layout (16 rows per key, contiguous).
+//
+// One row block per wave (RB = 1) for the small stages, where more waves shorten the whole; two for
+// stages that fill the card anyway, which then read S_D once per 32 rows.
+//
+// k-step q of the MFMA uses key 4 q + lk, and FP32 values are formed as in gemm_kernel: bitwise the
+// same in FP32.  Final stage in ms, tiles -> this: Heisenberg L=32 m=128 FP64 0.071 -> 0.015; Hubbard
+// L=64 m=1024 0.099 -> 0.036; TwoU1 L=16 m=301 FP32 0.254 -> 0.113; SU2U1 L=16 m=256 BF16X3 0.636 -> 0.163;
+// L=24 m=1000 FP64 3.67 -> 3.14, BF16X3 2.40 -> 2.02 (its tasks of at most 32 rows: 1.0 and 0.8 before).
+constexpr int FD = 2;
+
+template <int MODE, typename TB, int RB, int WK, bool TRA>
+__global__ __launch_bounds__(FT) __attribute__((amdgpu_waves_per_eu(2)))
+void f_wave_kernel(const GemmTask* __restrict__ tasks, uint32_t n_tasks, const GemmSeg* __restrict__ segs,
+                   Bases bases, GemmTables tables, const uint32_t* __restrict__ tile_task) {
+    typedef typename FsTraits<MODE>::T T;
+    typedef typename FsTraits<MODE>::Acc Acc;
+    constexpr int WCOL = 4 / WK, PB = FK + (MODE == MODE_F64 ? 2 : 4);
+    __shared__ __align__(16) T sb[4][16][PB];
+    __shared__ T sr[WK > 1 ? 4 : 1][WK > 1 ? RB * 256 : 1];
+    const uint32_t* __restrict__ maps = tables.maps;
+    const GemmUnit* __restrict__ units = tables.units;
+    const double* __restrict__ scales = tables.scales;
+
+    const uint32_t tile = xcd_tile_cyclic<4>(blockIdx.x, gridDim.x);
+    const GemmTask tk = tasks[f_task_of(tasks, n_tasks, tile_task, tile)];
+    const uint32_t M = tk.M, N = tk.N;
+    const uint32_t local = tile - tk.tile_begin;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int l16 = lane & 15, lk = lane >> 4;
+    const int part = wave % WK;
+    const uint32_t m0 = (local / tk.tiles_n) * (16 * RB), n0 = (local % tk.tiles_n) * (16 * WCOL) + (wave / WK) * 16;
+    if (WK == 1 && n0 >= N) return;   // WK > 1: one column block per workgroup, n0 < N
+
+    // ---- the wave's steps: [t0, t1) of the chain
+    uint32_t total = 0;
+    for (uint32_t s = tk.seg0; s < tk.seg1; ++s) total += (segs[s].K + FK - 1) / FK;
+    const uint32_t t0 = total * part / WK, t1 = total * (part + 1) / WK;
+
+    Acc acc[RB];
+#pragma unroll
+    for (int i = 0; i < RB; ++i) acc[i] = Acc{0, 0, 0, 0};
+
+    if (t0 < t1) {
+        uint32_t am[RB];
+#pragma unroll
+        for (int i = 0; i < RB; ++i) am[i] = min(m0 + uint32_t(16 * i + l16), M - 1);
+        const uint32_t bn = min(n0 + uint32_t(lane >> 2), N - 1);
+        const int b_k = 4 * (lane & 3);
+        const uint32_t unit = maps[tk.colunit + bn];
+
+        // cursor of the lookups: segment, first key of the step, steps left
+        uint32_t sgi = tk.seg0, k0 = 0, left = t1 - t0;
+        {
+            uint32_t skip = t0;
+            while (true) {
+                const uint32_t n = (segs[sgi].K + FK - 1) / FK;
+                if (skip < n) break;
+                skip -= n;
+                ++sgi;
+            }
+            k0 = skip * FK;
+        }
+        GemmSeg sg = segs[sgi];
+        uint32_t inv = 0;   // ceil(2^32 / bbh): k / bbh = mulhi(k, inv) for k, bbh < 2^16
+        auto magic = [&]() { inv = sg.bbh > 1 ? 0xffffffffu / sg.bbh + 1u : 0u; };
+        auto div = [&](uint32_t k) { return sg.bbh > 1 ? __umulhi(k, inv) : k; };
+        magic();
+        GemmUnit U = units[sg.units + unit], Un = U;   // of the current and of the next segment
+        auto fetch_unit = [&]() { Un = units[segs[min(sgi + 1, tk.seg1 - 1)].units + unit]; };
+        fetch_unit();
+
+        // a step looked up: B's map entries and offsets within the blocks, A's addresses
+        struct Look {
+            uint32_t row[4], kin[4];
+            const TB* col;
+            uint32_t ld;
+            bool ok;
+            const double* a;
+            uint32_t lda, K, k0;
+            uint32_t arow[TRA ? 4 : 1];   // A offset of key 4 q + lk of a transposed block, and its scale
+            double sc[TRA ? 4 : 1];
+            bool tra;
+            double alpha;
+        } lo;
+        auto look = [&]() {
+            lo.K = sg.K;
+            lo.k0 = k0;
+            lo.ok = U.valid != 0;
+            lo.ld = U.ld;
+            lo.col = reinterpret_cast<const TB*>(bases.p[sg.b_base]) + sg.b_off + U.src + uint64_t(sg.bbh) * (bn - U.col0);
+            lo.a = bases.p[sg.a_base] + sg.a_off;
+            lo.lda = sg.lda;
+            lo.alpha = sg.alpha;
+            lo.tra = TRA && sg.amap != MAP_NONE;
+            const uint32_t um = lo.ok ? U.map : 0u;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const uint32_t k = min(k0 + uint32_t(b_k + e), sg.K - 1), j = div(k);
+                lo.kin[e] = k - j * sg.bbh;
+                lo.row[e] = maps[lo.ok ? um + j : 0u];
+            }
+            if constexpr (TRA) {
+                if (lo.tra) {
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const uint32_t k = min(k0 + uint32_t(4 * q + lk), sg.K - 1), j = div(k);
+                        lo.arow[q] = maps[sg.amap + j] + (k - j * sg.bbh);
+                        lo.sc[q] = scales[sg.ascale + j];
+                    }
+                }
+            }
+        };
+        auto advance = [&]() {   // to the next step (at the last: stays)
+            if (left <= 1) return;
+            --left;
+            k0 += FK;
+            if (k0 >= sg.K) {
+                sg = segs[++sgi];
+                k0 = 0;
+                magic();
+                U = Un;
+                fetch_unit();
+            }
+        };
+        struct Set {   // a step's loads
+            TB b[4];
+            double a[RB][4];
+            T sc[TRA ? 4 : 1];
+            uint32_t K, k0;
+            bool ok;
+        } set[FD];
+        auto load = [&](Set& s) {
+            s.K = lo.K;
+            s.k0 = lo.k0;
+            s.ok = lo.ok;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const uint64_t o = uint64_t(lo.row[e]) * lo.ld + lo.kin[e];
+                s.b[e] = lo.col[lo.ok ? o : 0ull];
+            }
+            if (TRA && lo.tra) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    s.sc[TRA ? q : 0] = T(lo.alpha * lo.sc[TRA ? q : 0]);
+#pragma unroll
+                    for (int i = 0; i < RB; ++i) s.a[i][q] = lo.a[lo.arow[TRA ? q : 0] + uint64_t(am[i]) * lo.lda];
+                }
+            } else {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const uint64_t k = min(lo.k0 + uint32_t(4 * q + lk), lo.K - 1);
+                    if (TRA || q == 0) s.sc[TRA ? q : 0] = T(lo.alpha);
+#pragma unroll
+                    for (int i = 0; i < RB; ++i) s.a[i][q] = lo.a[am[i] + k * lo.lda];
+                }
+            }
+        };
+        T(*wb)[PB] = sb[wave];
+        auto step = [&](Set& s) {
+            T x[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[e] = s.ok && s.k0 + b_k + e < s.K ? T(s.b[e]) : T(0);
+            if constexpr (MODE == MODE_F32) {
+                *reinterpret_cast<float4*>(&wb[lane >> 2][b_k]) = float4{x[0], x[1], x[2], x[3]};
+            } else {
+                *reinterpret_cast<double2*>(&wb[lane >> 2][b_k]) = double2{x[0], x[1]};
+                *reinterpret_cast<double2*>(&wb[lane >> 2][b_k + 2]) = double2{x[2], x[3]};
+            }
+            T a[RB][4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int i = 0; i < RB; ++i) {
+                    a[i][q] = T(s.a[i][q]) * s.sc[TRA ? q : 0];
+                    if (s.k0 + 4 * q + lk >= s.K) a[i][q] = T(0);
+                }
+            load(s);      // the set is free: the step looked up last
+            advance();
+            look();
+            wave_fence();
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const T b = wb[l16][4 * q + lk];
+#pragma unroll
+                for (int i = 0; i < RB; ++i) {
+                    if constexpr (MODE == MODE_F64)
+                        acc[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i][q], b, acc[i], 0, 0, 0);
+                    else
+                        acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][q], b, acc[i], 0, 0, 0);
+                }
+            }
+            wave_fence();
+        };
+        look();
+#pragma unroll
+        for (int d = 0; d < FD; ++d) {
+            load(set[d]);
+            advance();
+            look();
+        }
+        uint32_t t = t0;
+        while (true) {
+#pragma unroll
+            for (int d = 0; d < FD; ++d) {
+                step(set[d]);
+                if (++t == t1) break;
+            }
+            if (t == t1) break;
+        }
+    }
+
+    // ---- sum of the parts in wave order, then C (FP64)
+    if constexpr (WK > 1) {
+#pragma unroll
+        for (int i = 0; i < RB; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) sr[wave][(i * 4 + r) * 64 + lane] = acc[i][r];
+        __syncthreads();
+        if (part) return;
+#pragma unroll
+        for (int i = 0; i < RB; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int w = 1; w < WK; ++w) acc[i][r] += sr[wave + w][(i * 4 + r) * 64 + lane];
+    }
+    double* __restrict__ C = bases.p[tk.c_base] + tk.c_off;
+    const uint32_t gn = n0 + l16;
+    if (gn < N) {
+#pragma unroll
+        for (int i = 0; i < RB; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const uint32_t gm = m0 + 16 * i + (MODE == MODE_F64 ? 4 * r + lk : 4 * lk + r);
+                if (gm < M) C[gm + uint64_t(gn) * tk.ldc] = double(acc[i][r]);
+            }
+    }
+}
+
 template <int BM>
 hipError_t launch_f_tile(hipStream_t st, int mode, const GemmTask* tasks, uint32_t n_tasks, const GemmSeg* segs,
                          uint32_t n_tiles, Bases bases, GemmTables tb, const uint32_t* tile_task) {
@@ -358,6 +616,31 @@ hipError_t launch_f_tile(hipStream_t st, int mode, const GemmTask* tasks, uint32
 }
 
 }  // namespace
+
+hipError_t launch_f_wave(hipStream_t st, int mode, int row_blocks, bool transposed, const GemmTask* tasks, uint32_t n_tasks,
+                         const GemmSeg* segs, uint32_t n_tiles, Bases bases, GemmTables tb, const uint32_t* tile_task) {
+    if (n_tiles == 0) return hipSuccess;
+#define MQ_F_WAVE(M_, TB_, RB_, WK_, TRA_)                                                                    \
+    hipLaunchKernelGGL((f_wave_kernel<M_, TB_, RB_, WK_, TRA_>), dim3(n_tiles), dim3(FT), 0, st, tasks, n_tasks, \
+                       segs, bases, tb, tile_task)
+#define MQ_F_WAVE_TR(M_, TB_, RB_, WK_)                    \
+    if (transposed) MQ_F_WAVE(M_, TB_, RB_, WK_, true);    \
+    else MQ_F_WAVE(M_, TB_, RB_, WK_, false)
+    if (mode == MODE_F64 && row_blocks == 1) {
+        MQ_F_WAVE_TR(MODE_F64, double, 1, 4);
+    } else if (mode == MODE_F64 && row_blocks == 2) {
+        MQ_F_WAVE_TR(MODE_F64, double, 2, 4);
+    } else if (mode == MODE_F32 && row_blocks == 1) {
+        MQ_F_WAVE_TR(MODE_F32, float, 1, 1);
+    } else if (mode == MODE_F32 && row_blocks == 2) {
+        MQ_F_WAVE_TR(MODE_F32, float, 2, 1);
+    } else {
+        return hipErrorInvalidValue;
+    }
+#undef MQ_F_WAVE_TR
+#undef MQ_F_WAVE
+    return hipGetLastError();
+}
 
 hipError_t launch_f_unit(hipStream_t st, int cfg, int mode, const GemmTask* tasks, uint32_t n_tasks, const GemmSeg* segs,
                          uint32_t n_tiles, Bases bases, GemmTables tb, const uint32_t* tile_task) {

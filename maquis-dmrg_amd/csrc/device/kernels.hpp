@@ -222,6 +222,13 @@ hipError_t launch_t_stream(hipStream_t st, int cls, int mode, bool c_float, cons
 // C double); same tables, tiles per task and results as launch_gemm with that cfg.
 hipError_t launch_f_unit(hipStream_t st, int cfg, int mode, const GemmTask* tasks, uint32_t n_tasks, const GemmSeg* segs,
                          uint32_t n_tiles, Bases bases, GemmTables tb, const uint32_t* tile_task);
+// The same tasks (any size) on the wave form: MODE_F64 (tiles of 16 row_blocks x 16, 4 waves share the K
+// chain) or MODE_F32 (A double, B float; tiles of 16 row_blocks x 64, bitwise gemm_kernel's result);
+// row_blocks 1 or 2.  Every segment's K and bbh in [1, 2^16).  Tiles are numbered column tile fastest
+// (GemmTask::tiles_n).  transposed: some segment has a block-remapped transposed A.
+constexpr uint32_t F_WAVE_COLS_F64 = 16, F_WAVE_COLS_F32 = 64;
+hipError_t launch_f_wave(hipStream_t st, int mode, int row_blocks, bool transposed, const GemmTask* tasks, uint32_t n_tasks,
+                         const GemmSeg* segs, uint32_t n_tiles, Bases bases, GemmTables tb, const uint32_t* tile_task);
 constexpr int GATHER_THREADS = 256;
 constexpr int GATHER_CHUNK = 1024;   // elements per workgroup
 constexpr int RED_BLOCKS = 512;      // fixed grid of the deterministic reductions
