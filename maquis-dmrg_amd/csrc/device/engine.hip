@@ -417,6 +417,23 @@ struct GemmStage {
     Stream wave64, wave32;
     bool wave64_all = false, wave_tr = false;
 
+    // FP64 stages of stacked tasks that read A through the units' block map: the boundary steps' final
+    // stage, all of it on its own kernel
+    Stream step_final;
+    static bool step_task(const GemmTask& t, const std::vector<GemmSeg>& segs, const std::vector<GemmRow>& rows,
+                          const std::vector<uint32_t>& maps) {
+        if (t.rowunit == MAP_NONE || t.beta || !t.M || !t.N || t.seg1 <= t.seg0) return false;
+        for (uint32_t k = t.seg0; k < t.seg1; ++k) {
+            const GemmSeg& g = segs[k];
+            if (g.amap == MAP_NONE || g.bmap != MAP_NONE || g.units != MAP_NONE || !g.K ||
+                g.trans_a != segs[t.seg0].trans_a || g.trans_b != segs[t.seg0].trans_b)
+                return false;
+        }
+        for (uint32_t m = 0; m < t.M; m += 16)
+            if (rows[maps[t.rowunit + m / 16]].cmap != MAP_NONE) return false;
+        return true;
+    }
+
     static bool wave_task(const GemmTask& t, const std::vector<GemmSeg>& segs) {
         if (t.rowunit != MAP_NONE || t.colunit == MAP_NONE || t.beta || t.m_off || t.cmap != MAP_NONE || !t.M || !t.N ||
             t.seg1 <= t.seg0)
@@ -451,9 +468,20 @@ struct GemmStage {
     }
     // streamed: take the streamed T kernel for the tasks it suits (plans whose T stage writes T_D in its
     // own type: all but the library S stage's)
-    void build(const std::vector<GemmTask>& tasks, const std::vector<GemmSeg>& segs, bool streamed = false) {
+    // f64_only: the stage runs in FP64 alone (boundary steps)
+    void build(const std::vector<GemmTask>& tasks, const std::vector<GemmSeg>& segs, const std::vector<GemmRow>& rows,
+               const std::vector<uint32_t>& maps, bool streamed, bool f64_only) {
         static const bool generic = std::getenv("MQ_T_GENERIC") != nullptr;
         all = tasks;
+        if (f64_only && !generic) {
+            bool every = !all.empty();
+            for (const auto& t : all) every = every && step_task(t, segs, rows, maps);
+            if (every) {
+                step_final.tasks.swap(all);
+                step_final.number(STEP_FINAL_TILE, STEP_FINAL_TILE);
+                step_final.finish();
+            }
+        }
         cls_of.assign(all.size(), -1);
         if (streamed && !generic)
             for (size_t i = 0; i < all.size(); ++i) cls_of[i] = int8_t(stream_class(all[i], segs));
@@ -564,8 +592,15 @@ struct GemmStage {
         for (auto& s : stream) s.upload_all(st);
         wave64.upload_all(st);
         wave32.upload_all(st);
+        step_final.upload_all(st);
     }
     void run(hipStream_t st, int mode, const char* types, Bases b, GemmTables tb) const {
+        if (step_final.tiles) {
+            MQ_REQUIRE(mode == MODE_F64, "boundary steps run in FP64");
+            HIPCHK(launch_step_final(st, step_final.d_tasks.as<GemmTask>(), uint32_t(step_final.tasks.size()),
+                                     d_segs.as<GemmSeg>(), step_final.tiles, b, tb, step_final.table()));
+            return;
+        }
         for (int c = 0; c < T_STREAM_N; ++c) {
             const Stream& s = stream[c];
             if (!s.tiles) continue;
@@ -855,10 +890,11 @@ struct StagePlan {
     DevBuf d_maps, d_units, d_scales, d_rows, d_zero_ws, d_zero_bf, d_regions, d_small, d_src_off, d_alpha;
     uint64_t sizes[N_BASES] = {0, 0, 0, 0, 0, 0};   // element counts of each base for validation
 
-    void finish_tables() {
-        gT.build(t_tasks, t_segs, bsr_on);
-        gF.build(f_tasks, f_segs);
-        gU.build(u_tasks, u_segs);
+    // f64_only: the plan is a boundary step's
+    void finish_tables(bool f64_only = false) {
+        gT.build(t_tasks, t_segs, rows, maps, bsr_on, false);
+        gF.build(f_tasks, f_segs, rows, maps, false, f64_only);
+        gU.build(u_tasks, u_segs, rows, maps, false, false);
         red.finish();
         std::vector<GatherRegion> big;
         for (const auto& r : regions) {
@@ -3963,7 +3999,7 @@ static int step_grouped(mq_ctx* ctx, int kind, const mq_site_desc* site, const m
                 continue;
             }
             P.blas = ctx->blas;
-            P.finish_tables();
+            P.finish_tables(true);
             P.sizes[BASE_WS] = P.ws_elems;
             P.sizes[BASE_IN] = P.sizes[BASE_BRA] = L.rp_total;
             P.sizes[BASE_OUT] = nb->total;

@@ -216,6 +216,12 @@ constexpr uint32_t T_STREAM_KMAX[T_STREAM_N] = {64, 144, 288}, T_STREAM_ROWS[T_S
 hipError_t launch_t_stream(hipStream_t st, int cls, int mode, bool c_float, const GemmTask* tasks, uint32_t n_tasks,
                            const GemmSeg* segs, uint32_t n_tiles, uint32_t strip, Bases bases, GemmTables tb,
                            const uint32_t* tile_task);
+// FP64 stacked tasks whose segments address A through the units' block map (amap, bldk; no B remaps, no
+// column map), one orientation (trans_a, trans_b) per task: the final stage of the boundary steps.
+// Tiles of STEP_FINAL_TILE x STEP_FINAL_TILE, column tile fastest (GemmTask::tiles_n).
+constexpr uint32_t STEP_FINAL_TILE = 64;
+hipError_t launch_step_final(hipStream_t st, const GemmTask* tasks, uint32_t n_tasks, const GemmSeg* segs, uint32_t n_tiles,
+                             Bases bases, GemmTables tb, const uint32_t* tile_task);
 // Final-stage tasks of tile configuration cfg (GEMM_CFG_128x128 or GEMM_CFG_64x64) whose segments
 // all read B through column units (no row units, no B block map, no beta, m_off 0) on the lean
 // kernel of f_stage.hip: MODE_F64 (all double), MODE_F32 or MODE_BF16X3 (A double, B float,

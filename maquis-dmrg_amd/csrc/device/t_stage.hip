@@ -656,6 +656,161 @@ hipError_t launch_t_stream_mode(hipStream_t st, int cls, const GemmTask* tasks, 
     return hipGetLastError();
 }
 
+// The final stage of the boundary steps (FP64): one stacked task per new cohort, its blocks the row
+// units, K segments over the physical states, each reading every unit's S_D slab through its block map
+// (GemmSeg::amap):
+//
+//   right step  A(m, k) = S[.. + i + k lda] (rows contiguous), B(k, n) = bra[.. + n + k ldb]
+//   left step   A(m, k) = S[.. + i lda + k] (keys contiguous), B(k, n) = bra[.. + k + n ldb]
+//
+// What bounds it: the bra side N is one sector, so a task is a tall product that reads S_D about once; the
+// generic kernel spent its time on per-element addresses and on loads whose neighbouring lanes are
+// different columns, one step ahead.  Here a thread stages 4 keys of one row of A and of one column of
+// B, dealt so that neighbouring lanes read neighbouring addresses in either orientation, two steps
+// ahead; 4 waves of 16 x 64 skip the column blocks beyond N alike.  SU2U1 L=30 m=1500 right step, final
+// stage: 10.0 -> 3.6 ms; L=24 m=1000 left step: 2.8 -> 1.1 ms.
+constexpr int RS_BM = 64, RS_BN = 64, RS_P = TK + 2;
+__global__ __launch_bounds__(TT) __attribute__((amdgpu_waves_per_eu(3)))
+void step_final_kernel(const GemmTask* __restrict__ tasks, uint32_t n_tasks, const GemmSeg* __restrict__ segs,
+                       Bases bases, GemmTables tables, const uint32_t* __restrict__ tile_task) {
+    __shared__ __align__(16) double sa[2][RS_BM][RS_P], sb[2][RS_BN][RS_P];
+    const uint32_t* __restrict__ maps = tables.maps;
+    const GemmRow* __restrict__ rows = tables.rows;
+
+    const uint32_t tile = xcd_tile_cyclic<16>(blockIdx.x, gridDim.x);
+    const GemmTask tk = tasks[task_of(tasks, n_tasks, tile_task, tile)];
+    const uint32_t M = tk.M, N = tk.N;
+    const uint32_t local = tile - tk.tile_begin;   // column tile fastest: a row panel's tiles share its S_D
+    const uint32_t m0 = (local / tk.tiles_n) * RS_BM, n0 = (local % tk.tiles_n) * RS_BN;
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int l16 = lane & 15, lk = lane >> 4;
+
+    // the orientation is one for all segments of a task
+    const bool ta = segs[tk.seg0].trans_a != 0, tb = segs[tk.seg0].trans_b != 0;
+    const int a_m = ta ? tid >> 2 : tid & 63, a_k = 4 * (ta ? tid & 3 : tid >> 6);
+    const int b_n = tb ? tid & 63 : tid >> 2, b_k = 4 * (tb ? tid >> 6 : tid & 3);
+    uint32_t a_i, a_j;
+    double a_rs;
+    {
+        const uint32_t m = min(m0 + uint32_t(a_m), M - 1);
+        const GemmRow& R = rows[maps[tk.rowunit + m / 16]];
+        a_i = min(m - R.row0, R.nrows - 1);
+        a_j = R.jblk;
+        a_rs = R.a_scale;
+    }
+    const uint32_t bn = min(n0 + uint32_t(b_n), N - 1);
+    const int nj = int(min((N - n0 + 15) / 16, uint32_t(RS_BN / 16)));   // column blocks inside N (uniform)
+
+    // cursor over the steps of all segments; a segment's row and column addresses
+    uint32_t sgi = tk.seg0, k0 = 0;
+    GemmSeg sg = segs[sgi];
+    const double *a_row = nullptr, *b_col = nullptr;
+    auto begin_seg = [&]() {
+        a_row = bases.p[sg.a_base] + sg.a_off + uint64_t(maps[sg.amap + a_j]) * sg.bldk + uint64_t(a_i) * (ta ? sg.lda : 1u);
+        b_col = bases.p[sg.b_base] + sg.b_off + uint64_t(bn) * (tb ? 1u : sg.ldb);
+    };
+    auto advance = [&]() {   // to the next step; false (and stays) at the last
+        if (k0 + TK < sg.K) {
+            k0 += TK;
+            return true;
+        }
+        if (sgi + 1 >= tk.seg1) return false;
+        sg = segs[++sgi];
+        k0 = 0;
+        begin_seg();
+        return true;
+    };
+    struct Stage {
+        double a[4], b[4];
+        double sc;
+        uint32_t k0, K;
+    };
+    auto load = [&](Stage& s) {   // keys beyond the segment read its last one
+        s.k0 = k0;
+        s.K = sg.K;
+        s.sc = a_rs * sg.alpha;
+        const uint64_t ask = ta ? 1u : sg.lda, bsk = tb ? sg.ldb : 1u;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            s.a[e] = a_row[uint64_t(min(k0 + uint32_t(a_k + e), sg.K - 1)) * ask];
+            s.b[e] = b_col[uint64_t(min(k0 + uint32_t(b_k + e), sg.K - 1)) * bsk];
+        }
+    };
+    auto store = [&](const Stage& s, int buf) {
+        double x[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] = s.k0 + a_k + e < s.K ? s.a[e] * s.sc : 0.0;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            *reinterpret_cast<double2*>(&sa[buf][a_m][a_k + 2 * h]) = double2{x[2 * h], x[2 * h + 1]};
+            *reinterpret_cast<double2*>(&sb[buf][b_n][b_k + 2 * h]) = double2{s.b[2 * h], s.b[2 * h + 1]};
+        }
+    };
+    d4 acc[RS_BN / 16];
+#pragma unroll
+    for (int j = 0; j < RS_BN / 16; ++j) acc[j] = d4{0, 0, 0, 0};
+    auto compute = [&](int buf) {
+        double a[4];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const double2 x = *reinterpret_cast<const double2*>(&sa[buf][16 * wave + l16][4 * lk + 2 * h]);
+            a[2 * h] = x.x, a[2 * h + 1] = x.y;
+        }
+#pragma unroll
+        for (int j = 0; j < RS_BN / 16; ++j) {
+            if (j >= nj) break;
+            double b[4];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const double2 x = *reinterpret_cast<const double2*>(&sb[buf][16 * j + l16][4 * lk + 2 * h]);
+                b[2 * h] = x.x, b[2 * h + 1] = x.y;
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[e], b[e], acc[j], 0, 0, 0);
+        }
+    };
+    // compute step t from one buffer, step t + 1 in registers, step t + 2's loads issued (past the last
+    // step the loads repeat it, unused)
+    begin_seg();
+    Stage ga, gb;
+    load(ga);
+    bool has = advance();
+    load(gb);
+    store(ga, 0);
+    __syncthreads();
+    while (true) {
+        const bool next = has && advance();
+        load(ga);
+        compute(0);
+        if (!has) break;
+        store(gb, 1);
+        __syncthreads();
+        has = next && advance();
+        load(gb);
+        compute(1);
+        if (!next) break;
+        store(ga, 0);
+        __syncthreads();
+    }
+
+    // ---- the wave's 16 rows lie in one unit
+    const uint32_t mb = m0 + 16 * wave;
+    if (mb >= M) return;
+    const GemmRow R = rows[maps[tk.rowunit + mb / 16]];
+    double* __restrict__ C = bases.p[tk.c_base] + tk.c_off + R.c_src;
+#pragma unroll
+    for (int j = 0; j < RS_BN / 16; ++j) {
+        const uint32_t gn = n0 + 16 * j + l16;
+        if (gn >= N) continue;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const uint32_t li = mb + 4 * r + lk - R.row0;
+            if (li < R.nrows) C[uint64_t(gn) * R.ldc + uint64_t(li) * R.c_si] = acc[j][r];
+        }
+    }
+}
+
 template <int BM>
 hipError_t launch_t_tile(hipStream_t st, int mode, bool c_float, const GemmTask* tasks, uint32_t n_tasks,
                          const GemmSeg* segs, uint32_t n_tiles, Bases bases, GemmTables tb, const uint32_t* tile_task) {
@@ -674,6 +829,13 @@ hipError_t launch_t_tile(hipStream_t st, int mode, bool c_float, const GemmTask*
 }
 
 }  // namespace
+
+hipError_t launch_step_final(hipStream_t st, const GemmTask* tasks, uint32_t n_tasks, const GemmSeg* segs, uint32_t n_tiles,
+                             Bases bases, GemmTables tb, const uint32_t* tile_task) {
+    if (n_tiles == 0) return hipSuccess;
+    hipLaunchKernelGGL(step_final_kernel, dim3(n_tiles), dim3(TT), 0, st, tasks, n_tasks, segs, bases, tb, tile_task);
+    return hipGetLastError();
+}
 
 hipError_t launch_t_stream(hipStream_t st, int cls, int mode, bool c_float, const GemmTask* tasks, uint32_t n_tasks,
                            const GemmSeg* segs, uint32_t n_tiles, uint32_t strip, Bases bases, GemmTables tb,

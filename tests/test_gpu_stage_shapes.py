@@ -61,3 +61,36 @@ def test_sigma_stages_match_oracle(eng, model, L, site, m):
             plan.apply(psi, out, precision=prec)
             eng.sync()
             assert torch.equal(first, out)
+
+
+@pytest.mark.parametrize("kind", ["left", "right"])
+@pytest.mark.parametrize("model,L,site,m", [("heisenberg", 16, 7, 150), ("heisenberg", 12, 1, 64), ("hubbard", 12, 5, 301),
+                                            ("qc", 8, 3, 77), ("qc_su2", 10, 4, 131), ("qc_su2", 12, 8, 57)])
+def test_steps_match_oracle(eng, kind, model, L, site, m):
+    """Boundary steps over one site: sectors below and above one 64-row / 64-column tile, odd sizes."""
+    from mqdmrg.engine import MpoDesc, SiteDesc
+    from mqdmrg import mps
+    from mqdmrg.symmetry import SiteLayout
+    ws = SyntheticSite(model, L, site, m, seed=L + m)
+    k = site if kind == "left" else site + 1
+    index = ws.left_index if kind == "left" else ws.right_index
+    lay = SiteLayout(ws.bonds[k], ws.basis.phys, ws.bonds[k + 1])
+    sd, md = SiteDesc(ws.basis.sym, ws.bonds[k], ws.basis.phys, ws.bonds[k + 1]), MpoDesc(ws.mpo[k])
+    coh = ws.random_cohorts(index)
+    hb = O.HostBoundary(index, [x if x is not None else np.zeros(0) for x in coh])
+    bra, ket = mps.random_site_vector(lay, ws.rng), mps.random_site_vector(lay, ws.rng)
+    d = lambda x: torch.from_numpy(np.ascontiguousarray(x)).to("cuda:0")  # noqa: E731
+    b = E.DeviceBoundary.upload(eng, index, coh)
+    if kind == "left":
+        ref = O.left_step(sd, md, mps.rp_to_lp(lay, bra), ket, hb, True)
+        new = E.left_step(eng, sd, md, d(mps.rp_to_lp(lay, bra)), d(ket), b)
+    else:
+        ref = O.right_step(sd, md, bra, ket, hb, True)
+        new = E.right_step(eng, sd, md, d(bra), d(ket), b)
+    num = den = 0.0
+    for x, y in zip(new.download(), ref.cohorts):
+        if len(y):
+            num += float(np.sum((x - y) ** 2))
+            den += float(np.sum(y ** 2))
+    print("%s %s L=%d site=%d m=%d: %.2e" % (kind, model, L, site, m, np.sqrt(num / den)), flush=True)
+    assert np.sqrt(num / den) <= RTOL[E.PREC_F64]
