@@ -20,6 +20,7 @@
 #include <cstdlib>
 #include <cstdio>
 #include <cstring>
+#include <exception>
 #include <functional>
 #include <limits>
 #include <map>
@@ -78,14 +79,22 @@ static void (*g_release_pools)() = nullptr;
 struct DevBuf {
     void* p = nullptr;
     size_t bytes = 0;
+    bool view = false;   // a part of another buffer (TableUpload, the W tiles), not freed here
     DevBuf() = default;
     DevBuf(const DevBuf&) = delete;
     DevBuf& operator=(const DevBuf&) = delete;
     ~DevBuf() { release(); }
     void release() {
-        if (p) (void)hipFree(p);
+        if (p && !view) (void)hipFree(p);
         p = nullptr;
         bytes = 0;
+        view = false;
+    }
+    void set_view(void* q, size_t n) {
+        release();
+        p = n ? q : nullptr;
+        bytes = n;
+        view = n != 0;
     }
     void alloc(size_t n) {
         release();
@@ -109,6 +118,7 @@ struct DevBuf {
     void swap(DevBuf& o) {
         std::swap(p, o.p);
         std::swap(bytes, o.bytes);
+        std::swap(view, o.view);
     }
     // allocation cleared to zero bits: library GEMMs called with beta = 0 may still read their C
     // operand (0 * NaN of stale memory is NaN), so workspaces never hold non-finite garbage
@@ -129,7 +139,71 @@ void upload(DevBuf& b, const std::vector<T>& v, hipStream_t st) {
     }
 }
 
+// One nonzero of a group's W_D: column n (N key position), row k (K key position), value.
+struct WEntry {
+    uint32_t n, k;
+    double v;
+};
+// Allocator whose resize() leaves trivial elements uninitialised (the nonzero lists are filled
+// completely right after they are sized; clearing hundreds of MB first would cost as much)
+template <class T> struct UninitAlloc : std::allocator<T> {
+    template <class U> struct rebind { using other = UninitAlloc<U>; };
+    UninitAlloc() = default;
+    template <class U> UninitAlloc(const UninitAlloc<U>&) {}
+    template <class U> void construct(U* q) { ::new (static_cast<void*>(q)) U; }
+    template <class U, class... A> void construct(U* q, A&&... a) { ::new (static_cast<void*>(q)) U(std::forward<A>(a)...); }
+};
+typedef std::vector<WEntry, UninitAlloc<WEntry>> WList;
+// one nonzero of W_D of group g at (column n, row k), from one MPO row
+struct RawW { uint32_t g, n, k; double v; };
+struct LowerScratch {
+    static constexpr size_t MAX_BYTES = size_t(1) << 30;
+    std::vector<std::vector<RawW>> raw;   // per MPO row
+    std::vector<WList> wg;                // per group
+    size_t bytes() const {
+        size_t n = 0;
+        for (const auto& r : raw) n += r.capacity() * sizeof(RawW);
+        for (const auto& w : wg) n += w.capacity() * sizeof(WEntry);
+        return n;
+    }
+};
+
+
 inline uint64_t align32(uint64_t x) { return round_up(x, 32); }
+
+// f(i) for i < n over the host threads; an exception thrown in one is rethrown here.
+template <class F>
+void parallel_for(size_t n, F&& f) {
+    std::exception_ptr err;
+#pragma omp parallel for schedule(dynamic, 1)
+    for (int64_t i = 0; i < int64_t(n); ++i) {
+        try {
+            f(size_t(i));
+        } catch (...) {
+#pragma omp critical(mq_parallel_for)
+            err = std::current_exception();
+        }
+    }
+    if (err) std::rethrow_exception(err);
+}
+
+// A plan's or step's host tables, collected and sent as one copy from pinned memory into one
+// allocation (the tables become views of it): some thirty allocations and pageable copies cost more
+// than the tables' bytes.
+struct TableUpload {
+    struct Item {
+        DevBuf* b;
+        const void* src;
+        size_t n, off;
+    };
+    std::vector<Item> items;
+    size_t total = 0;
+    template <class T>
+    void operator()(DevBuf& b, const std::vector<T>& v) {
+        items.push_back({&b, v.data(), v.size() * sizeof(T), total});
+        total += (v.size() * sizeof(T) + 255) & ~size_t(255);
+    }
+};
 
 }  // namespace
 
@@ -193,7 +267,7 @@ struct mq_ctx {
     // one plan per site, and allocating and releasing tens of GB per site costs more than the
     // site's products.  A slot keeps the largest buffer returned to it; a request it cannot serve
     // allocates 25% headroom, so that the slightly larger plans of the next sites still fit.
-    enum PoolKind { POOL_WS, POOL_PART, POOL_WS32, POOL_BF, POOL_KINDS };
+    enum PoolKind { POOL_WS, POOL_PART, POOL_WS32, POOL_BF, POOL_TABLES, POOL_W, POOL_ENT, POOL_KINDS };
     DevBuf pool[POOL_KINDS];
     // pinned host staging of the dense MPO matrices W_D of the plan (or step chunk) being lowered;
     // grows, and is reused by the next lowering once the previous upload has been synchronized
@@ -215,6 +289,23 @@ struct mq_ctx {
             std::memset(wd_host + o, 0, size_t(std::min<int64_t>(chunk, int64_t(n) - o)) * sizeof(double));
         return wd_host;
     }
+    // pinned staging of a plan's or step's tables (TableUpload); grows, reused by the next one
+    char* tab_host = nullptr;
+    size_t tab_cap = 0;
+    char* tab_stage(size_t n) {
+        if (n > tab_cap) {
+            if (tab_host) (void)hipHostFree(tab_host);
+            tab_host = nullptr;
+            tab_cap = 0;
+            const size_t cap = (n + n / 4 + (size_t(1) << 20) - 1) & ~((size_t(1) << 20) - 1);
+            HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&tab_host), cap, hipHostMallocDefault));
+            tab_cap = cap;
+        }
+        return tab_host;
+    }
+    // host lists of the lowering (lower_sigma_grouped), kept between plans: hundreds of MB of first
+    // touches per plan otherwise.  Taken while in use, put back if within the bound.
+    LowerScratch lower_scratch;
     void pool_put(PoolKind kind, DevBuf& b) {
         if (!b.p) return;
         if (pool[kind].bytes < b.bytes) pool[kind].swap(b);
@@ -402,10 +493,11 @@ struct GemmStage {
             tiles = uint32_t(tile);
         }
         void finish() { tile_task = tiles_to_tasks(tasks, tiles); }
-        void upload_all(hipStream_t st) {
+        template <class Up>
+        void upload_all(Up& up) {
             if (tasks.empty()) return;
-            upload(d_tasks, tasks, st);
-            upload(d_tile_task, tile_task, st);
+            up(d_tasks, tasks);
+            up(d_tile_task, tile_task);
         }
         const uint32_t* table() const { return tile_task.empty() ? nullptr : d_tile_task.as<uint32_t>(); }
         uint64_t device_bytes() const { return d_tasks.bytes + d_tile_task.bytes; }
@@ -558,7 +650,9 @@ struct GemmStage {
             w->finish();
         }
     }
-    void upload_all(const std::vector<GemmSeg>& segs, hipStream_t st) {
+    // up(buffer, table): TableUpload, or an upload of its own (the autotuner's rebuilds)
+    template <class Up>
+    void upload_all(const std::vector<GemmSeg>& segs, Up&& up) {
         static const bool generic = std::getenv("MQ_T_GENERIC") != nullptr;
         static const bool generic_f = std::getenv("MQ_F_GENERIC") != nullptr;
         for (int c = 0; c < GEMM_N_CFG; ++c) {
@@ -584,15 +678,15 @@ struct GemmStage {
                 stacked[c] = stacked[c] && ok;
             }
         }
-        upload(d_segs, segs, st);
+        if (!all.empty() || !step_final.tasks.empty()) up(d_segs, segs);
         for (int c = 0; c < GEMM_N_CFG; ++c) {
-            upload(d_tasks[c], cfg[c], st);
-            upload(d_tile_task[c], tile_task[c], st);
+            up(d_tasks[c], cfg[c]);
+            up(d_tile_task[c], tile_task[c]);
         }
-        for (auto& s : stream) s.upload_all(st);
-        wave64.upload_all(st);
-        wave32.upload_all(st);
-        step_final.upload_all(st);
+        for (auto& s : stream) s.upload_all(up);
+        wave64.upload_all(up);
+        wave32.upload_all(up);
+        step_final.upload_all(up);
     }
     void run(hipStream_t st, int mode, const char* types, Bases b, GemmTables tb) const {
         if (step_final.tiles) {
@@ -666,11 +760,11 @@ struct GatherSet {
         }
         chunks = ch;
     }
-    void upload_all(hipStream_t st) {
-        upload(d_regions, regions, st);
-        upload(d_small, small, st);
-        upload(d_src_off, src_off, st);
-        upload(d_alpha, alpha, st);
+    void upload_all(TableUpload& up) {
+        up(d_regions, regions);
+        up(d_small, small);
+        up(d_src_off, src_off);
+        up(d_alpha, alpha);
     }
     void run(hipStream_t st, double* src, double* dst) const {
         if (empty()) return;
@@ -731,7 +825,6 @@ struct StagePlan {
         uint64_t* ent_pos = nullptr;
         double* ent_val = nullptr;
         uint64_t n_ent = 0;
-        bool uploaded = false;
         uint64_t tiles = 0;
         uint64_t flops = 0;             // MFMA flops of the visited tiles (unpadded)
         bool narrow = true;             // every task's T_D step window fits 32-bit byte offsets
@@ -890,8 +983,7 @@ struct StagePlan {
     DevBuf d_maps, d_units, d_scales, d_rows, d_zero_ws, d_zero_bf, d_regions, d_small, d_src_off, d_alpha;
     uint64_t sizes[N_BASES] = {0, 0, 0, 0, 0, 0};   // element counts of each base for validation
 
-    // f64_only: the plan is a boundary step's
-    void finish_tables(bool f64_only = false) {
+    void finish_tables() {
         gT.build(t_tasks, t_segs, rows, maps, bsr_on, false);
         gF.build(f_tasks, f_segs, rows, maps, false, f64_only);
         gU.build(u_tasks, u_segs, rows, maps, false, false);
@@ -988,10 +1080,11 @@ struct StagePlan {
     }
     void validate() const {
         auto gemm = [&](const std::vector<GemmTask>& tasks, const std::vector<GemmSeg>& segs, bool split) {
-            for (const auto& t : tasks) {
+            parallel_for(tasks.size(), [&](size_t ti) {
+                const GemmTask& t = tasks[ti];
                 if (t.rowunit != MAP_NONE) {
                     check_stacked(t, segs, split);
-                    continue;
+                    return;
                 }
                 MQ_REQUIRE(t.ldc >= t.M || t.N <= 1, "ldc < M");
                 if (t.cmap == MAP_NONE) {
@@ -1061,7 +1154,7 @@ struct StagePlan {
                         check_in(g.b_base, g.b_off, extent(t.N, g.K, g.ldb), "B^T");
                     }
                 }
-            }
+            });
         };
         gemm(t_tasks, t_segs, split_t);
         gemm(f_tasks, f_segs, false);
@@ -1108,50 +1201,84 @@ struct StagePlan {
                 for (uint32_t t = r.t0; t < r.t1; ++t) check_in(BASE_WS, src_off[t], uint64_t(r.R) * r.C, "T slab");
             }
     }
-    void upload_all(hipStream_t st) {
-        gT.upload_all(t_segs, st);
-        gF.upload_all(f_segs, st);
-        gU.upload_all(u_segs, st);
-        if (bsr_on && !bsr.uploaded) {   // once: the host copy of the nonzeros is released after it
-            upload(bsr.d_tasks, bsr.tasks, st);
-            upload(bsr.d_runs, bsr.runs, st);
-            upload(bsr.d_tile_cols, bsr.tile_cols, st);
+    // Tables and W tiles to the device, on ctx's stream (the caller synchronizes before the host tables
+    // go).  give_back returns the buffers to the context's pools.
+    DevBuf tables, wtiles;
+    bool f64_only = false;   // a boundary step: no reduced-precision tiles
+    void give_back(mq_ctx* ctx) {
+        ctx->pool_put(mq_ctx::POOL_TABLES, tables);
+        ctx->pool_put(mq_ctx::POOL_W, wtiles);
+    }
+    void upload_all(mq_ctx* ctx) {
+        hipStream_t st = ctx->stream;
+        TableUpload up;
+        gT.upload_all(t_segs, up);
+        gF.upload_all(f_segs, up);
+        gU.upload_all(u_segs, up);
+        if (bsr_on) {
+            up(bsr.d_tasks, bsr.tasks);
+            up(bsr.d_runs, bsr.runs);
+            up(bsr.d_tile_cols, bsr.tile_cols);
+        }
+        up(d_regions, regions);
+        up(d_small, small);
+        up(d_src_off, src_off);
+        up(d_alpha, alpha);
+        up(d_maps, maps);
+        up(d_units, units);
+        up(d_scales, scales);
+        up(d_rows, rows);
+        up(d_zero_ws, zero_ws);
+        up(d_zero_bf, zero_bf);
+        red.upload_all(up);
+        ctx->take(mq_ctx::POOL_TABLES, tables, std::max<size_t>(up.total, 256), false);
+        HIPCHK(hipStreamSynchronize(st));   // no earlier copy reads the staging any more
+        char* stage = ctx->tab_stage(std::max<size_t>(up.total, 256));
+        const int64_t chunk = int64_t(1) << 20;
+        std::vector<std::pair<const TableUpload::Item*, size_t>> parts;
+        for (const auto& it : up.items) {
+            it.b->set_view(tables.as<char>() + it.off, it.n);
+            for (size_t o = 0; o < it.n; o += size_t(chunk)) parts.push_back({&it, o});
+        }
+#pragma omp parallel for schedule(static) if (parts.size() > 8)
+        for (int64_t i = 0; i < int64_t(parts.size()); ++i) {
+            const TableUpload::Item& it = *parts[i].first;
+            const size_t o = parts[i].second;
+            std::memcpy(stage + it.off + o, static_cast<const char*>(it.src) + o, std::min(size_t(chunk), it.n - o));
+        }
+        if (up.total) HIPCHK(hipMemcpyAsync(tables.p, stage, up.total, hipMemcpyHostToDevice, st));
+        if (bsr_on) {
             // the W tiles in the three arithmetics: FP64 zero-filled and the nonzeros scattered into
             // it; FP32 and the bf16 split of the FP32 value converted on the device
-            const uint64_t nw = bsr.tiles * uint64_t(S_BSR_TILE_N) * S_BSR_TILE_K;
-            bsr.d_w64.alloc(std::max<uint64_t>(nw, 1) * sizeof(double));
+            const uint64_t nw = std::max<uint64_t>(bsr.tiles * uint64_t(S_BSR_TILE_N) * S_BSR_TILE_K, 32);
+            ctx->take(mq_ctx::POOL_W, wtiles, nw * (f64_only ? 8 : 16), false);
+            bsr.d_w64.set_view(wtiles.p, nw * sizeof(double));
             HIPCHK(launch_fill(st, bsr.d_w64.as<double>(), nw, 0.0));
             if (bsr.n_ent) {
-                DevBuf d_pos, d_val;
-                d_pos.alloc(bsr.n_ent * sizeof(uint64_t));
-                d_val.alloc(bsr.n_ent * sizeof(double));
-                HIPCHK(hipMemcpyAsync(d_pos.p, bsr.ent_pos, bsr.n_ent * sizeof(uint64_t), hipMemcpyHostToDevice, st));
-                HIPCHK(hipMemcpyAsync(d_val.p, bsr.ent_val, bsr.n_ent * sizeof(double), hipMemcpyHostToDevice, st));
-                HIPCHK(launch_scatter(st, bsr.n_ent, d_pos.as<uint64_t>(), d_val.as<double>(), bsr.d_w64.as<double>()));
-                HIPCHK(hipStreamSynchronize(st));   // before the entry buffers are freed and the staging reused
+                DevBuf ent;   // positions, then values
+                ctx->take(mq_ctx::POOL_ENT, ent, 2 * bsr.n_ent * sizeof(uint64_t), false);
+                uint64_t* pos = ent.as<uint64_t>();
+                double* val = ent.as<double>() + bsr.n_ent;
+                HIPCHK(hipMemcpyAsync(pos, bsr.ent_pos, bsr.n_ent * sizeof(uint64_t), hipMemcpyHostToDevice, st));
+                HIPCHK(hipMemcpyAsync(val, bsr.ent_val, bsr.n_ent * sizeof(double), hipMemcpyHostToDevice, st));
+                HIPCHK(launch_scatter(st, bsr.n_ent, pos, val, bsr.d_w64.as<double>()));
+                // the entry staging is reused by the next lowering, which this stream's work precedes
+                // only for the device: wait for the copies
+                HIPCHK(hipStreamSynchronize(st));
+                ctx->pool_put(mq_ctx::POOL_ENT, ent);
             }
-            bsr.d_w32.alloc(std::max<uint64_t>(nw, 1) * sizeof(float));
-            bsr.d_whi.alloc(std::max<uint64_t>(nw, 1) * sizeof(uint16_t));
-            bsr.d_wlo.alloc(std::max<uint64_t>(nw, 1) * sizeof(uint16_t));
-            HIPCHK(launch_split_tiles(st, bsr.d_w64.as<double>(), nw, bsr.d_w32.as<float>(), bsr.d_whi.as<uint16_t>(),
-                                      bsr.d_wlo.as<uint16_t>()));
-            HIPCHK(hipStreamSynchronize(st));   // the host copy is released below
+            if (!f64_only) {
+                char* w = wtiles.as<char>();
+                bsr.d_w32.set_view(w + nw * 8, nw * sizeof(float));
+                bsr.d_whi.set_view(w + nw * 12, nw * sizeof(uint16_t));
+                bsr.d_wlo.set_view(w + nw * 14, nw * sizeof(uint16_t));
+                HIPCHK(launch_split_tiles(st, bsr.d_w64.as<double>(), nw, bsr.d_w32.as<float>(), bsr.d_whi.as<uint16_t>(),
+                                          bsr.d_wlo.as<uint16_t>()));
+            }
             bsr.ent_pos = nullptr;
             bsr.ent_val = nullptr;
             bsr.n_ent = 0;
-            bsr.uploaded = true;
         }
-        upload(d_regions, regions, st);
-        upload(d_small, small, st);
-        upload(d_src_off, src_off, st);
-        upload(d_alpha, alpha, st);
-        upload(d_maps, maps, st);
-        upload(d_units, units, st);
-        upload(d_scales, scales, st);
-        upload(d_rows, rows, st);
-        upload(d_zero_ws, zero_ws, st);
-        upload(d_zero_bf, zero_bf, st);
-        red.upload_all(st);
     }
     // the four stages of an application: zero-fill, T GEMM, middle (gather or S GEMM), final GEMM.
     // mode != MODE_F64 (grouped plans only): T_D, S_D and W_D are FP32 in a float workspace.
@@ -1554,6 +1681,7 @@ int mq_ctx_destroy(mq_ctx* ctx) {
         if (ctx->fork_ev) (void)hipEventDestroy(ctx->fork_ev);
         ctx->pool_clear();
         if (ctx->wd_host) (void)hipHostFree(ctx->wd_host);
+        if (ctx->tab_host) (void)hipHostFree(ctx->tab_host);
         g_contexts.erase(std::remove(g_contexts.begin(), g_contexts.end(), ctx), g_contexts.end());
         if (ctx->blas) (void)rocblas_destroy_handle(ctx->blas);
         if (ctx->lt) (void)hipblasLtDestroy(ctx->lt);
@@ -1659,10 +1787,11 @@ int reshape(mq_ctx* ctx, const mq_site_desc* site, const double* src, double* ds
             for (uint32_t t = r.t0; t < r.t1; ++t)
                 MQ_REQUIRE(P.src_off[t] + uint64_t(r.R) * r.C <= n_src, "reshape src out of range");
         });
-        P.upload_all(ctx->stream);
+        P.upload_all(ctx);
         HIPCHK(launch_fill(ctx->stream, dst, n_dst, 0.0));
         P.run_gather(ctx->stream, const_cast<double*>(src), dst);
         HIPCHK(hipStreamSynchronize(ctx->stream));   // tables are freed on return
+        P.give_back(ctx);
     });
 }
 }  // namespace
@@ -2122,22 +2251,6 @@ struct GroupedStep {
     uint32_t lo = 0, hi = 0xffffffffu;
 };
 
-// One nonzero of a group's W_D: column n (N key position), row k (K key position), value.
-struct WEntry {
-    uint32_t n, k;
-    double v;
-};
-// Allocator whose resize() leaves trivial elements uninitialised (the nonzero lists are filled
-// completely right after they are sized; clearing hundreds of MB first would cost as much)
-template <class T> struct UninitAlloc : std::allocator<T> {
-    template <class U> struct rebind { using other = UninitAlloc<U>; };
-    UninitAlloc() = default;
-    template <class U> UninitAlloc(const UninitAlloc<U>&) {}
-    template <class U> void construct(U* q) { ::new (static_cast<void*>(q)) U; }
-    template <class U, class... A> void construct(U* q, A&&... a) { ::new (static_cast<void*>(q)) U(std::forward<A>(a)...); }
-};
-typedef std::vector<WEntry, UninitAlloc<WEntry>> WList;
-
 // Pattern-class order of one group's keys (see lower_sigma_grouped): rows k and columns n of W_D
 // are classed by a hash of their nonzero index lists; classes are ordered by size (largest first),
 // then by their first key; the all-zero class goes last.  W holds the group's nonzeros in an order
@@ -2379,10 +2492,16 @@ void lower_sigma_grouped(mq_plan* p, const SiteLayout& site, const Mpo& W, uint6
         for (auto b : jb) MQ_REQUIRE(b != MQ_NONE, "cohort with unmapped stored block");
         return jb;
     };
-    // ---- pairs and groups
-    for (uint32_t lb = 0; lb < left_i.size(); ++lb) {
+    // ---- pairs and groups: every sector pair's key lists in parallel, then the groups in pair order
+    struct Cand {
+        uint32_t rb;
+        std::vector<uint32_t> K, N;
+    };
+    std::vector<std::vector<Cand>> cand(left_i.size());
+    parallel_for(left_i.size(), [&](size_t lbi) {
+        const uint32_t lb = uint32_t(lbi);
         Charge lc_in = left_i.charges[lb];
-        if (rstep && (lb < step->lo || lb >= step->hi)) continue;
+        if (rstep && (lb < step->lo || lb >= step->hi)) return;
         for (uint32_t rb = 0; rb < right_i.size(); ++rb) {
             Charge rc_out = right_i.charges[rb];
             if (lstep && (rb < step->lo || rb >= step->hi)) continue;
@@ -2411,8 +2530,14 @@ void lower_sigma_grouped(mq_plan* p, const SiteLayout& site, const Mpo& W, uint6
                 else
                     add_keys(N, NI, NI.cohort_index(lc_in, rc_out - phys_i.charges[s]), s, true);
             }
-            if (K.empty() || N.empty()) continue;
-            Charge d = rc_out - lc_in;
+            if (!K.empty() && !N.empty()) cand[lb].push_back({rb, std::move(K), std::move(N)});
+        }
+    });
+    for (uint32_t lb = 0; lb < left_i.size(); ++lb) {
+        Charge lc_in = left_i.charges[lb];
+        for (Cand& c : cand[lb]) {
+            const uint32_t rb = c.rb;
+            Charge d = right_i.charges[rb] - lc_in;
             auto ins = group_of.emplace(std::make_pair(d.key(), sy.spin(lc_in)), uint32_t(G.groups.size()));
             if (ins.second) {
                 G.groups.emplace_back();
@@ -2429,10 +2554,10 @@ void lower_sigma_grouped(mq_plan* p, const SiteLayout& site, const Mpo& W, uint6
             pr.m_off = g.M;
             g.M += uint64_t(left_i.sizes[lb]) * right_i.sizes[rb];
             // keys for now; numbered within the group once every pair is known
-            for (auto k : K) g.kpos[k] = 0;
-            for (auto n : N) g.npos[n] = 0;
-            pr.kk = std::move(K);
-            pr.nn = std::move(N);
+            for (auto k : c.K) g.kpos[k] = 0;
+            for (auto n : c.N) g.npos[n] = 0;
+            pr.kk = std::move(c.K);
+            pr.nn = std::move(c.N);
             g.pairs.push_back(uint32_t(G.pairs.size()));
             G.pair_of[uint64_t(lb) << 32 | rb] = uint32_t(G.pairs.size());
             G.pairs.push_back(std::move(pr));
@@ -2494,7 +2619,6 @@ void lower_sigma_grouped(mq_plan* p, const SiteLayout& site, const Mpo& W, uint6
     const bool sparse_w = !adjoint;
     const bool bsr = !adjoint && s_sparse_enabled();
     double* const wd = bsr ? nullptr : p->ctx->wd_stage(wd_elems);
-    std::vector<WList> wg(sparse_w ? G.groups.size() : 0);
     trace_phase("lower: key order, layout");
     if (g_trace) {
         uint64_t tk = 0, tn = 0, tm = 0;
@@ -2505,9 +2629,14 @@ void lower_sigma_grouped(mq_plan* p, const SiteLayout& site, const Mpo& W, uint6
     }
     struct AdjEntry { uint32_t t; uint64_t w; double c; };
     std::vector<AdjEntry> adj;
-    // one nonzero of W_D of group g at (column n, row k), from one MPO row
-    struct RawW { uint32_t g, n, k; double v; };
-    std::vector<std::vector<RawW>> raw(sparse_w ? W.row_dim : 0);
+    LowerScratch scratch;   // the context's lists, put back (below) unless something fails
+    std::swap(scratch, p->ctx->lower_scratch);
+    std::vector<std::vector<RawW>>& raw = scratch.raw;
+    if (sparse_w && raw.size() < W.row_dim) raw.resize(W.row_dim);
+    for (auto& r : raw) r.clear();
+    std::vector<WList>& wg = scratch.wg;
+    if (sparse_w && wg.size() < G.groups.size()) wg.resize(G.groups.size());
+    for (auto& w : wg) w.clear();
     // ---- W_D: for every MPO entry, its (k, n) in each group holding both keys.  The groups of
     // a K key are listed per key (CSR over the dense key numbering)
     std::vector<uint32_t> kg_off(size_t(G.nkeys) + 1, 0);
@@ -2654,7 +2783,7 @@ void lower_sigma_grouped(mq_plan* p, const SiteLayout& site, const Mpo& W, uint6
         // b2 (keys are b-major; a row's cells ascend in b2; a cell emits in (k, n) order), so for
         // every k its columns n, and for every n its rows k, come in ascending order, the order
         // reorder_group_keys hashes them in.
-        const size_t ng = G.groups.size(), nb = raw.size();
+        const size_t ng = G.groups.size(), nb = W.row_dim;
         std::vector<uint64_t> off(nb * ng, 0);   // per (b1, g): entries, then first slot
 #pragma omp parallel for schedule(dynamic, 16)
         for (int b1 = 0; b1 < int(nb); ++b1)
@@ -2671,7 +2800,6 @@ void lower_sigma_grouped(mq_plan* p, const SiteLayout& site, const Mpo& W, uint6
 #pragma omp parallel for schedule(dynamic, 16)
         for (int b1 = 0; b1 < int(nb); ++b1) {
             for (const RawW& e : raw[b1]) wg[e.g][off[size_t(b1) * ng + e.g]++] = {e.n, e.k, e.v};
-            std::vector<RawW>().swap(raw[b1]);
         }
     }
     trace_phase("lower: W_D");
@@ -2777,7 +2905,17 @@ void lower_sigma_grouped(mq_plan* p, const SiteLayout& site, const Mpo& W, uint6
         // ---- T stage of the left step: X(pair (lb_bra, rb_ket), key (b1, s, ss)) = L_b1(lb_bra, lb_ket)
         // ket(lb_ket)[:, columns (s, ss, rb_ket)], stacked per left cohort and (s, ss): its blocks b1
         // are row units sharing the ket columns
-        for (uint32_t lb = 0; lb < left_i.size(); ++lb)
+        // (a row unit per block of every cohort and state: built per bra sector in parallel, appended in order)
+        struct Piece {
+            std::vector<GemmTask> tasks;
+            std::vector<GemmSeg> segs;
+            std::vector<GemmRow> rows;
+            std::vector<uint32_t> maps;
+        };
+        std::vector<Piece> pieces(left_i.size());
+        parallel_for(left_i.size(), [&](size_t lbi) {
+            const uint32_t lb = uint32_t(lbi);
+            Piece& Q = pieces[lb];
             for (uint32_t lbk = 0; lbk < left_i.size(); ++lbk) {
                 const uint32_t cl = LI.cohort_index(left_i.charges[lb], left_i.charges[lbk]);
                 const uint32_t lsb = left_i.sizes[lb], lsk = left_i.sizes[lbk];
@@ -2820,20 +2958,45 @@ void lower_sigma_grouped(mq_plan* p, const SiteLayout& site, const Mpo& W, uint6
                             R.ldc = lsb;
                             R.c_si = 1;
                             R.cmap = MAP_NONE;
-                            unit_of_blk.insert(unit_of_blk.end(), (lsb + 15) / 16, uint32_t(P.rows.size()));
-                            P.rows.push_back(R);
+                            unit_of_blk.insert(unit_of_blk.end(), (lsb + 15) / 16, uint32_t(Q.rows.size()));
+                            Q.rows.push_back(R);
                         }
                         const uint32_t Mt = uint32_t(unit_of_blk.size()) * 16;
                         const uint64_t col0 = rpb(s, rb) + uint64_t(ss) * rs;
-                        GemmTask& t = add_gemm(P.t_tasks, P.t_segs, BASE_WS, 0, Mt, rs, Mt,
+                        GemmTask& t = add_gemm(Q.tasks, Q.segs, BASE_WS, 0, Mt, rs, Mt,
                                                {seg(BASE_LEFT, 0, 1, false, BASE_IN, site.rp_offset[lbk] + col0 * lsk,
                                                     lsk, false, lsk)});
                         t.cbw = rs;
-                        t.rowunit = uint32_t(P.maps.size());
-                        P.maps.insert(P.maps.end(), unit_of_blk.begin(), unit_of_blk.end());
+                        t.rowunit = uint32_t(Q.maps.size());
+                        Q.maps.insert(Q.maps.end(), unit_of_blk.begin(), unit_of_blk.end());
                     }
                 }
             }
+        });
+        std::vector<std::array<size_t, 4>> at(pieces.size() + 1);   // first task, segment, row, map entry of a piece
+        at[0] = {P.t_tasks.size(), P.t_segs.size(), P.rows.size(), P.maps.size()};
+        for (size_t i = 0; i < pieces.size(); ++i)
+            at[i + 1] = {at[i][0] + pieces[i].tasks.size(), at[i][1] + pieces[i].segs.size(), at[i][2] + pieces[i].rows.size(),
+                         at[i][3] + pieces[i].maps.size()};
+        const auto& end = at.back();
+        MQ_REQUIRE(end[1] < (1ull << 32) && end[2] < (1ull << 32) && end[3] < (1ull << 32), "step tables too large");
+        P.t_tasks.resize(end[0]);
+        P.t_segs.resize(end[1]);
+        P.rows.resize(end[2]);
+        P.maps.resize(end[3]);
+        parallel_for(pieces.size(), [&](size_t i) {
+            Piece& Q = pieces[i];
+            for (auto& t : Q.tasks) {
+                t.seg0 += uint32_t(at[i][1]);
+                t.seg1 += uint32_t(at[i][1]);
+                t.rowunit += uint32_t(at[i][3]);
+            }
+            for (auto& m : Q.maps) m += uint32_t(at[i][2]);   // row units only
+            std::copy(Q.tasks.begin(), Q.tasks.end(), P.t_tasks.begin() + at[i][0]);
+            std::copy(Q.segs.begin(), Q.segs.end(), P.t_segs.begin() + at[i][1]);
+            std::copy(Q.rows.begin(), Q.rows.end(), P.rows.begin() + at[i][2]);
+            std::copy(Q.maps.begin(), Q.maps.end(), P.maps.begin() + at[i][3]);
+        });
     }
     trace_phase("lower: T stage");
     if (g_trace)
@@ -2894,7 +3057,6 @@ void lower_sigma_grouped(mq_plan* p, const SiteLayout& site, const Mpo& W, uint6
         P.bsr.ent_pos = reinterpret_cast<uint64_t*>(stage);
         P.bsr.ent_val = stage + cap;
         add_bsr_groups(P.bsr, G.groups, wg, g_trace ? &info : nullptr);
-        std::vector<WList>().swap(wg);
         P.bsr_on = true;
         for (size_t gi = 0; gi < info.size(); ++gi) {
             const auto& g = G.groups[gi];
@@ -2905,6 +3067,7 @@ void lower_sigma_grouped(mq_plan* p, const SiteLayout& site, const Mpo& W, uint6
         }
         trace_phase("lower: S tiles");
     }
+    if (scratch.bytes() <= LowerScratch::MAX_BYTES) std::swap(scratch, p->ctx->lower_scratch);
     for (auto& L : P.lib) {   // B' regions after the A' regions
         L.bfb_off = P.bf_elems;
         P.bf_elems += align32(3ull * L.K * L.N);
@@ -3304,7 +3467,7 @@ int mq_sigma_plan_create_from_schedule(mq_ctx* ctx, const mq_schedule_desc* sche
         P.sizes[BASE_RIGHT] = right->total;
         P.validate();
         p->ws.alloc_zeroed(std::max<uint64_t>(P.ws_elems, 32) * sizeof(double), ctx->stream);
-        P.upload_all(ctx->stream);
+        P.upload_all(ctx);
         HIPCHK(hipStreamSynchronize(ctx->stream));
         *out = p.release();
     });
@@ -3357,7 +3520,7 @@ int mq_sigma_plan_create_ex(mq_ctx* ctx, const mq_site_desc* site, const mq_mpo_
             HIPCHK(hipMemcpyAsync(p->ws.as<double>() + ws_init_off, ctx->wd_host, wd_elems * sizeof(double),
                                   hipMemcpyHostToDevice, ctx->stream));
         trace_phase("plan: workspaces");
-        P.upload_all(ctx->stream);
+        P.upload_all(ctx);
         HIPCHK(hipStreamSynchronize(ctx->stream));
         trace_phase("plan: upload");
         p->grouped = true;
@@ -3573,7 +3736,7 @@ int mq_plan_autotune(mq_plan* p, int precision, int* timed) {
             auto apply = [&](const TilePolicy& pol) {
                 G.policy = pol;
                 G.rebuild();
-                G.upload_all(*sr.segs, st);
+                G.upload_all(*sr.segs, [&](DevBuf& b, const auto& v) { upload(b, v, st); });
             };
             auto it = ctx->tuned.find(key);
             if (it != ctx->tuned.end()) {
@@ -3762,6 +3925,7 @@ int mq_plan_destroy(mq_plan* p) {
     return guarded([&] {
         if (p && p->ctx) {
             (void)hipStreamSynchronize(p->ctx->stream);
+            p->st.give_back(p->ctx);
             if (p->grouped) {   // the large workspaces go back to the context for the next plans
                 mq_ctx* c = p->ctx;
                 c->pool_put(mq_ctx::POOL_WS, p->ws);
@@ -3886,7 +4050,7 @@ static int left_step_schedule(mq_ctx* ctx, const mq_site_desc* site, const mq_mp
         P.sizes[BASE_OUT] = nb->total;
         P.sizes[BASE_LEFT] = left->total;
         P.validate();
-        P.upload_all(ctx->stream);
+        P.upload_all(ctx);
         ctx->step_ws.ensure(std::max<uint64_t>(ws, 32) * sizeof(double));
         Bases bs{};
         bs.p[BASE_WS] = ctx->step_ws.as<double>();
@@ -3896,6 +4060,7 @@ static int left_step_schedule(mq_ctx* ctx, const mq_site_desc* site, const mq_mp
         bs.p[BASE_BRA] = const_cast<double*>(bra_lp);
         P.run(ctx->stream, bs);
         HIPCHK(hipStreamSynchronize(ctx->stream));
+        P.give_back(ctx);
         *out = nb.release();
     });
 }
@@ -3932,7 +4097,7 @@ static int right_step_schedule(mq_ctx* ctx, const mq_site_desc* site, const mq_m
         P.sizes[BASE_OUT] = nb->total;
         P.sizes[BASE_RIGHT] = right->total;
         P.validate();
-        P.upload_all(ctx->stream);
+        P.upload_all(ctx);
         ctx->step_ws.ensure(std::max<uint64_t>(ws, 32) * sizeof(double));
         Bases bs{};
         bs.p[BASE_WS] = ctx->step_ws.as<double>();
@@ -3942,6 +4107,7 @@ static int right_step_schedule(mq_ctx* ctx, const mq_site_desc* site, const mq_m
         bs.p[BASE_BRA] = const_cast<double*>(bra_rp);
         P.run(ctx->stream, bs);
         HIPCHK(hipStreamSynchronize(ctx->stream));
+        P.give_back(ctx);
         *out = nb.release();
     });
 }
@@ -3999,13 +4165,14 @@ static int step_grouped(mq_ctx* ctx, int kind, const mq_site_desc* site, const m
                 continue;
             }
             P.blas = ctx->blas;
-            P.finish_tables(true);
+            P.f64_only = true;
+            P.finish_tables();
             P.sizes[BASE_WS] = P.ws_elems;
             P.sizes[BASE_IN] = P.sizes[BASE_BRA] = L.rp_total;
             P.sizes[BASE_OUT] = nb->total;
             P.sizes[kind == Schedule::LEFT ? BASE_LEFT : BASE_RIGHT] = bnd->total;
             P.validate();
-            P.upload_all(ctx->stream);
+            P.upload_all(ctx);
             // workspace: the context's pooled workspace (the site's sigma plan has returned it), taken
             // as it is with the block-sparse S stage (the grouped stages clear what they read
             // unwritten; cleared for library GEMMs) and grown between chunks when a chunk needs
@@ -4031,6 +4198,7 @@ static int step_grouped(mq_ctx* ctx, int kind, const mq_site_desc* site, const m
             trace_phase("step: workspace");
             P.run(ctx->stream, bs, MODE_F64);
             HIPCHK(hipStreamSynchronize(ctx->stream));   // the chunk's tables and the W_D staging are reused next
+            P.give_back(ctx);
             trace_phase("step: run");
         }
         ctx->pool_put(mq_ctx::POOL_WS, sws);   // back to the pool for the next site's sigma plan
