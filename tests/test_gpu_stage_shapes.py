@@ -26,6 +26,7 @@ SHAPES = [
     ("qc", 10, 1, 60),
     ("qc_su2", 10, 4, 131),
     ("qc_su2", 12, 8, 57),
+    ("qc_su2", 14, 6, 101),   # several 128-column panels, runs of odd and even numbers of key tiles
     ("heisenberg", 20, 9, 420),   # sectors of 65 to 144 and of more than 144
     ("heisenberg", 24, 11, 1100),   # and of more than 288
 ]
