@@ -166,19 +166,26 @@ hipError_t launch_zero_chunks(hipStream_t st, const ZeroChunk* chunks, uint32_t 
     return hipGetLastError();
 }
 
-__global__ void term_grad_kernel(uint32_t n_terms, const uint32_t* __restrict__ ptr, const uint64_t* __restrict__ idx,
-                                 const double* __restrict__ coef, const double* __restrict__ g, double* __restrict__ grad) {
-    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+// A wave per term: 64 entries at a time, then a tree over the lanes (fixed order).  The entries are
+// gathered from all over G: latency-bound, so many lanes at it (SU2U1 L=16 m=256: one thread per term
+// took 322 us for a handful of long terms, a tenth of the adjoint).
+constexpr int TERM_WAVES = 4;
+__global__ __launch_bounds__(64 * TERM_WAVES)
+void term_grad_kernel(uint32_t n_terms, const uint32_t* __restrict__ ptr, const uint64_t* __restrict__ idx,
+                      const double* __restrict__ coef, const double* __restrict__ g, double* __restrict__ grad) {
+    const uint32_t t = blockIdx.x * TERM_WAVES + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (t >= n_terms) return;
     double acc = 0.0;
-    for (uint32_t e = ptr[t]; e < ptr[t + 1]; ++e) acc += coef[e] * g[idx[e]];
-    grad[t] = acc;
+    for (uint64_t e = ptr[t] + uint64_t(lane), e1 = ptr[t + 1]; e < e1; e += 64) acc += coef[e] * g[idx[e]];
+#pragma unroll
+    for (int o = 32; o; o >>= 1) acc += __shfl_down(acc, o, 64);
+    if (lane == 0) grad[t] = acc;
 }
 hipError_t launch_term_grad(hipStream_t st, uint32_t n_terms, const uint32_t* ptr, const uint64_t* idx,
                             const double* coef, const double* g, double* grad) {
     if (n_terms == 0) return hipSuccess;
-    hipLaunchKernelGGL(term_grad_kernel, dim3((n_terms + 255) / 256), dim3(256), 0, st, n_terms, ptr, idx, coef, g,
-                       grad);
+    hipLaunchKernelGGL(term_grad_kernel, dim3((n_terms - 1) / TERM_WAVES + 1), dim3(64 * TERM_WAVES), 0, st, n_terms, ptr,
+                       idx, coef, g, grad);
     return hipGetLastError();
 }
 

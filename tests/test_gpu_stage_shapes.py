@@ -95,3 +95,23 @@ def test_steps_match_oracle(eng, kind, model, L, site, m):
             den += float(np.sum(y ** 2))
     print("%s %s L=%d site=%d m=%d: %.2e" % (kind, model, L, site, m, np.sqrt(num / den)), flush=True)
     assert np.sqrt(num / den) <= RTOL[E.PREC_F64]
+
+
+@pytest.mark.parametrize("model,L,site,m", [("heisenberg", 16, 7, 150), ("hubbard", 10, 7, 90), ("qc", 6, 2, 40),
+                                            ("qc_su2", 6, 2, 60)])
+def test_adjoint_matches_oracle(eng, model, L, site, m):
+    """Gradients per MPO term: terms of one entry and of thousands (64 entries a turn), groups of very
+    different sizes side by side, and a second gradient through the same plan."""
+    ws = SyntheticSite(model, L, site, m, seed=L + m)
+    Lc, Rc = ws.random_cohorts(ws.left_index), ws.random_cohorts(ws.right_index)
+    host = [O.HostBoundary(i, [x if x is not None else np.zeros(0) for x in c])
+            for i, c in ((ws.left_index, Lc), (ws.right_index, Rc))]
+    Lb, Rb = E.DeviceBoundary.upload(eng, ws.left_index, Lc), E.DeviceBoundary.upload(eng, ws.right_index, Rc)
+    plan = E.SigmaPlan(eng, ws.site_desc, ws.mpo_desc, Lb, Rb, algorithm=E.SIGMA_GROUPED, adjoint=True)
+    for _ in range(2):
+        psi_h = ws.random_psi()
+        ref = O.sigma_term_gradient(ws.site_desc, ws.mpo_desc, *host, psi_h)
+        g = plan.adjoint(torch.from_numpy(psi_h).to("cuda:0"))
+        err = np.linalg.norm(g - ref) / np.linalg.norm(ref)
+        print("adjoint %s L=%d site=%d m=%d: %.2e" % (model, L, site, m, err), flush=True)
+        assert err <= 10 * RTOL[E.PREC_F64]   # two products in a row and the sum over a term's entries
