@@ -3817,33 +3817,46 @@ int mq_sigma_adjoint(mq_plan* p, const double* psi, double* grad) {
         HIPCHK(launch_fill(st, ws + p->s_region0, p->s_region1 - p->s_region0, 0.0));
         P.run_u(st, b);
         // G_g = T_g^T U_g in the W_D layout: the derivative of psi . sigma with respect to W_D.  A group's
-        // product has a few tens of tiles: the groups run side by side on the side streams, each next one
-        // (largest first) on the stream with the least work (adjoint of SU2U1
-        // L=16 m=256: 3.8 ms one after another, 2.4 ms so)
+        // product has at most a few tens of tiles: from 6.5e6 flops a group on average the groups run side by
+        // side on the side streams, each next one (largest first) on the stream with the least work.  SU2U1,
+        // one after another / side by side: L=16 m=256 (1.1e8 a group) 3.45 / 2.37 ms, L=12 m=100 (8.6e6)
+        // 1.02 / 0.84, L=14 m=60 (4.6e6) 0.81 / 0.91, L=10 m=67 (2.8e6) 0.59 / 0.66: below it the launches
+        // bound both, and those to several streams cost more.
+        constexpr double FORK_FLOPS = 6.5e6;
         const double one = 1.0, zero = 0.0;
         double* G = p->adj_g.as<double>();
-        std::vector<size_t> order(P.lib.size());
-        std::iota(order.begin(), order.end(), size_t(0));
-        auto work = [&](size_t i) { return double(P.lib[i].M) * P.lib[i].N * P.lib[i].K + 1e6; };   // 1e6: a launch
-        std::stable_sort(order.begin(), order.end(), [&](size_t x, size_t y) { return work(x) > work(y); });
-        HIPCHK(hipEventRecord(ctx->fork_ev, st));
-        for (hipStream_t sd : ctx->side) HIPCHK(hipStreamWaitEvent(sd, ctx->fork_ev, 0));
-        try {
-            double load[mq_ctx::NSIDE] = {};
-            for (size_t i : order) {
-                const auto& g = P.lib[i];
-                const int k = int(std::min_element(load, load + mq_ctx::NSIDE) - load);
-                load[k] += work(i);
-                BLASCHK(rocblas_dgemm(ctx->side_blas[k], rocblas_operation_transpose, rocblas_operation_none, g.K, g.N, g.M, &one,
-                                      ws + g.a_off, g.lda, ws + g.c_off, g.ldc, &zero, G + (g.b_off - p->ws_init_off), g.K));
+        auto work = [&](size_t i) { return 2.0 * P.lib[i].M * P.lib[i].N * P.lib[i].K; };
+        auto product = [&](rocblas_handle h, size_t i) {
+            const auto& g = P.lib[i];
+            BLASCHK(rocblas_dgemm(h, rocblas_operation_transpose, rocblas_operation_none, g.K, g.N, g.M, &one, ws + g.a_off,
+                                  g.lda, ws + g.c_off, g.ldc, &zero, G + (g.b_off - p->ws_init_off), g.K));
+        };
+        double total = 0;
+        for (size_t i = 0; i < P.lib.size(); ++i) total += work(i);
+        if (total < FORK_FLOPS * double(P.lib.size())) {
+            BLASCHK(rocblas_set_stream(P.blas, st));
+            for (size_t i = 0; i < P.lib.size(); ++i) product(P.blas, i);
+        } else {
+            std::vector<size_t> order(P.lib.size());
+            std::iota(order.begin(), order.end(), size_t(0));
+            std::stable_sort(order.begin(), order.end(), [&](size_t x, size_t y) { return work(x) > work(y); });
+            HIPCHK(hipEventRecord(ctx->fork_ev, st));
+            for (hipStream_t sd : ctx->side) HIPCHK(hipStreamWaitEvent(sd, ctx->fork_ev, 0));
+            try {
+                double load[mq_ctx::NSIDE] = {};
+                for (size_t i : order) {
+                    const int k = int(std::min_element(load, load + mq_ctx::NSIDE) - load);
+                    load[k] += work(i) + 1e6;   // 1e6: a launch
+                    product(ctx->side_blas[k], i);
+                }
+                for (int k = 0; k < mq_ctx::NSIDE; ++k) {
+                    HIPCHK(hipEventRecord(ctx->side_ev[k], ctx->side[k]));
+                    HIPCHK(hipStreamWaitEvent(st, ctx->side_ev[k], 0));
+                }
+            } catch (...) {   // nothing of the plan stays in use on a side stream
+                for (hipStream_t sd : ctx->side) (void)hipStreamSynchronize(sd);
+                throw;
             }
-            for (int k = 0; k < mq_ctx::NSIDE; ++k) {
-                HIPCHK(hipEventRecord(ctx->side_ev[k], ctx->side[k]));
-                HIPCHK(hipStreamWaitEvent(st, ctx->side_ev[k], 0));
-            }
-        } catch (...) {   // nothing of the plan stays in use on a side stream
-            for (hipStream_t sd : ctx->side) (void)hipStreamSynchronize(sd);
-            throw;
         }
         // per term: the coefficients of its op entries against G
         HIPCHK(launch_term_grad(st, p->n_terms, p->d_adj_ptr.as<uint32_t>(), p->d_adj_idx.as<uint64_t>(),
