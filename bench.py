@@ -415,7 +415,7 @@ def main():
     else:
         # T and final stages: the lean MFMA kernels (and the generic grouped GEMM for other tile
         # shapes), FP32 accumulation in the reduced precisions
-        kernel = ("mq::t_stack_kernel (T stage)" if dom == "gemm_T" else "mq::f_unit_kernel (final stage)")
+        kernel = ("mq::t_stream_kernel (T stage)" if dom == "gemm_T" else "mq::f_unit_kernel (final stage)")
         peak_key = "f64" if report == "f64" else "f32"
     roof = {"kernel": kernel, "bound": "mfma", "achieved": achieved, "peak": PEAK_TFLOPS[peak_key],
             "unit": "TFLOP/s", "frac": achieved / PEAK_TFLOPS[peak_key], "traffic": None, "stage_ms": st,
