@@ -9,9 +9,9 @@
 // T_D rows (column-major, rows contiguous) straight into registers in the MFMA layout, since every wave
 // has rows of its own, and the compact W tiles, which all waves share, through LDS, double buffered.
 //
-// What bounds it: FP64 the MFMA rate (about 62 of the 73 TFLOP/s a large FP64 product reaches, counting the
-// zeros inside visited 16 x 16 blocks), BF16X3 the memory (24 GB of T_D and S_D once at L=30, 5.6 ms at
-// the copy rate).  A visited 16 x 128 tile is on average two thirds full by 16-column blocks; every wave
+// What bounds it: FP64 the MFMA rate (matrix units busy 80% of the time; 61 of the 73 TFLOP/s a large FP64
+// product reaches, counting the zeros inside visited 16 x 16 blocks), BF16X3 the memory (L=30:
+// 31 GB read, T_D about twice, and 8.4 GB written in 8.3 ms, 4.8 TB/s).  A visited 16 x 128 tile is on average two thirds full by 16-column blocks; every wave
 // spans the tile's 128 columns and skips the blocks without a nonzero (the same for every wave; adding a
 // zero product changes no bit), and the loads run two steps ahead.  S stage at SU2U1 L=30 m=1500: FP64
 // 49.8 ms with every block multiplied, 30.8 ms with blocks skipped, tiles dealt to the XCDs and T_D staged
@@ -83,9 +83,10 @@ template <> struct BsrTraits<MODE_F32> { typedef float T; typedef f4 Acc; };
 template <> struct BsrTraits<MODE_BF16X3> { typedef float T; typedef f4 Acc; };
 
 // One step's W tiles in LDS, [n][k].  FP64 / FP32 rows are padded by 16 bytes: 16-byte chunks are stored
-// whole and the MFMA reads (16 columns, 4 keys) meet no bank twice.  BF16X3: rows of 32 keys, 16-byte
+// whole.  FP64's reads meet banks twice at that stride (45% of the LDS cycles); rows of 17 doubles, read
+// without a conflict but stored by halves, were slower (L=30 m=1500: 27.1 against 26.4 ms).  BF16X3: rows of 32 keys, 16-byte
 // chunks of 8 keys, chunk c of row n at c ^ (n / 2 % 4): 8 lanes that read (or store) the same chunk of 8
-// consecutive rows meet 8 different chunks of the 32 banks.
+// consecutive rows meet 8 different chunks of the 32 banks (no conflict counted).
 template <int MODE> struct BsrSmem {
     typedef typename BsrTraits<MODE>::T T;
     T b[BN][BK + 16 / sizeof(T)];
