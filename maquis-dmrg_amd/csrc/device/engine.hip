@@ -1133,8 +1133,7 @@ struct StagePlan {
                         MQ_REQUIRE(uint64_t(g.units) + t.nunits <= units.size(), "unit table range");
                         const uint32_t nblk = g.K / g.bbh;
                         for (uint32_t u = 0; u < t.nunits; ++u) {
-                            const GemmUnit& U = units[g.units + u];
-                            if (!U.valid) continue;
+                            const GemmUnit& U = units[g.units + u];   // valid or not: its loads are masked, not left out
                             MQ_REQUIRE(U.col0 + ucols[u] <= t.N, "unit columns");
                             for (uint32_t n = U.col0; n < U.col0 + ucols[u]; ++n)
                                 MQ_REQUIRE(maps[t.colunit + n] == u, "unit columns are not contiguous");
@@ -3074,6 +3073,7 @@ void lower_sigma_grouped(mq_plan* p, const SiteLayout& site, const Mpo& W, uint6
         L.bfb_off = P.bf_elems;
         P.bf_elems += align32(3ull * L.K * L.N);
     }
+    uint64_t masked_elems = 0;   // extent of the masked loads of units without an S_D block
     if (sigma) {
         // ---- final stage: one task per output block lb_out (ls_out x all its columns), K segments over
         // the left cohorts (lc_out, lc_in).  The block's columns fall into units (s, ss2) of rs columns;
@@ -3118,6 +3118,12 @@ void lower_sigma_grouped(mq_plan* p, const SiteLayout& site, const Mpo& W, uint6
                         d.map = uint32_t(P.maps.size());
                         d.valid = 1;
                         for (uint32_t b1 : b1s) P.maps.push_back(g.nid(G.key(b1, U.s, U.ss)));
+                    } else {
+                        // no S_D block (a right boundary without the unit's cohorts): the kernels load it
+                        // all the same and mask the values, from column 0 of a block at the workspace's start
+                        d.map = uint32_t(P.maps.size());
+                        P.maps.insert(P.maps.end(), b1s.size(), 0u);
+                        masked_elems = std::max(masked_elems, uint64_t(left_i.sizes[lb_in]) * U.rs);
                     }
                     P.units.push_back(d);
                 }
@@ -3377,7 +3383,7 @@ void lower_sigma_grouped(mq_plan* p, const SiteLayout& site, const Mpo& W, uint6
     }
     // the block-sparse S stage reads 128 rows of every key column it visits (the rows of a short
     // panel past M are zeroed after loading): room for those past the last region
-    P.ws_elems = ws + (P.bsr_on ? S_BSR_TILE_M : 0);
+    P.ws_elems = std::max(ws + (P.bsr_on ? S_BSR_TILE_M : 0), align32(masked_elems));
     if (!sigma) return;
     // T and L reference flops now; the S part (a scan of W_D per pair) when first asked for
     p->flops = 0;

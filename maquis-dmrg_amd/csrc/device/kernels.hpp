@@ -109,6 +109,8 @@ struct GemmSeg {
     uint8_t a_base, b_base, trans_a, trans_b;
 };
 
+// valid == 0: the unit's B is zero; src, ld and map still describe addresses inside B's buffer, which the
+// kernels may read and mask
 struct GemmUnit {
     uint64_t src;
     uint32_t ld, map, col0, valid;

@@ -1,0 +1,75 @@
+"""Forms of the stage kernels and of the plans around them that the chains' ordinary sites do not
+reach: boundaries with cohorts left out, sectors beyond one tile of the step kernel, the adjoint's
+products side by side, wide groups, large stages."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as O
+from mqdmrg import engine as E
+from mqdmrg.capi import BIndex
+from mqdmrg.workloads import SyntheticSite
+
+pytestmark = pytest.mark.gpu
+
+RTOL = {E.PREC_F64: 1e-13, E.PREC_F32: 1e-5, E.PREC_BF16X3: 1e-4}
+
+
+@pytest.fixture(scope="module")
+def eng():
+    e = E.Engine(0)
+    yield e
+    e.close()
+
+
+def host_boundary(index, cohorts):
+    return O.HostBoundary(index, [x if x is not None else np.zeros(0) for x in cohorts])
+
+
+def check_sigma(eng, ws, left_index, right_index, label, min_bytes=0):
+    """sigma of a site with the given boundary indices against the oracle, in all three precisions."""
+    Lc, Rc = ws.random_cohorts(left_index), ws.random_cohorts(right_index)
+    psi_h = ws.random_psi()
+    ref = O.SigmaOracle(ws.site_desc, ws.mpo_desc, host_boundary(left_index, Lc), host_boundary(right_index, Rc)).apply(psi_h)
+    assert np.linalg.norm(ref) > 0
+    Lb, Rb = E.DeviceBoundary.upload(eng, left_index, Lc), E.DeviceBoundary.upload(eng, right_index, Rc)
+    plan = E.SigmaPlan(eng, ws.site_desc, ws.mpo_desc, Lb, Rb)
+    assert plan.workspace_bytes >= min_bytes
+    psi = torch.from_numpy(psi_h).to("cuda:0")
+    for prec, tol in RTOL.items():
+        print("%s precision %d" % (label, prec), flush=True)
+        out = torch.full_like(psi, float("nan"))
+        plan.apply(psi, out, precision=prec)
+        eng.sync()
+        err = np.linalg.norm(out.cpu().numpy() - ref) / np.linalg.norm(ref)
+        print("  relative error %.2e" % err, flush=True)
+        assert err <= tol
+    plan.close()
+
+
+def subset(index, keep):
+    """The boundary index with only the cohorts `keep`."""
+    keep = np.asarray(keep)
+    return BIndex(index.bra, index.ket, index.aux_dim, index.bra_pos[keep], index.ket_pos[keep], index.tr[keep],
+                  index.n_blocks[keep], index.offsets[keep], index.conj_scales[keep], index.transposes[keep])
+
+
+@pytest.mark.parametrize("model,L,site,m", [("heisenberg", 26, 12, 8192), ("heisenberg", 20, 9, 420), ("hubbard", 12, 5, 301),
+                                            ("qc", 10, 4, 150)])
+def test_right_boundary_with_one_sector(model, L, site, m):
+    """A right boundary that holds its smallest sector alone: most output columns then have no S_D block
+    in most segments (units the kernels load masked).  What T_D and S_D need is far smaller than a left
+    sector times a right one, the extent of such a unit's addresses: the workspace has to hold that."""
+    ws = SyntheticSite(model, L, site, m, seed=L + m)
+    idx = ws.right_index
+    diag = [c for c in range(idx.n_cohorts) if idx.bra_pos[c] == idx.ket_pos[c] and not idx.tr[c] and idx.cohort_size(c)]
+    small = min(diag, key=lambda c: idx.bra.sizes[idx.bra_pos[c]])
+    # the widest unit without an S_D block: left sector lb_out, one state of the right sector it meets
+    left, right = ws.left_index.bra, idx.bra
+    widest = max(right.sizes[r] for r in range(len(right.charges)) if r != idx.bra_pos[small])
+    eng = E.Engine(0)   # no workspace of an earlier plan
+    try:
+        check_sigma(eng, ws, ws.left_index, subset(idx, [small]), "%s L=%d site=%d m=%d" % (model, L, site, m),
+                    min_bytes=8 * widest * max(left.sizes))
+    finally:
+        eng.close()
