@@ -26,7 +26,7 @@ def host_boundary(index, cohorts):
     return O.HostBoundary(index, [x if x is not None else np.zeros(0) for x in cohorts])
 
 
-def check_sigma(eng, ws, left_index, right_index, label, min_bytes=0):
+def check_sigma(eng, ws, left_index, right_index, label):
     """sigma of a site with the given boundary indices against the oracle, in all three precisions."""
     Lc, Rc = ws.random_cohorts(left_index), ws.random_cohorts(right_index)
     psi_h = ws.random_psi()
@@ -34,7 +34,6 @@ def check_sigma(eng, ws, left_index, right_index, label, min_bytes=0):
     assert np.linalg.norm(ref) > 0
     Lb, Rb = E.DeviceBoundary.upload(eng, left_index, Lc), E.DeviceBoundary.upload(eng, right_index, Rc)
     plan = E.SigmaPlan(eng, ws.site_desc, ws.mpo_desc, Lb, Rb)
-    assert plan.workspace_bytes >= min_bytes
     psi = torch.from_numpy(psi_h).to("cuda:0")
     for prec, tol in RTOL.items():
         print("%s precision %d" % (label, prec), flush=True)
@@ -59,17 +58,14 @@ def subset(index, keep):
 def test_right_boundary_with_one_sector(model, L, site, m):
     """A right boundary that holds its smallest sector alone: most output columns then have no S_D block
     in most segments (units the kernels load masked).  What T_D and S_D need is far smaller than a left
-    sector times a right one, the extent of such a unit's addresses: the workspace has to hold that."""
+    sector times a right one, the extent of such a unit's addresses: the workspace has to hold that
+    too, or the plan's check of its tables, which leaves no unit out, refuses it."""
     ws = SyntheticSite(model, L, site, m, seed=L + m)
     idx = ws.right_index
     diag = [c for c in range(idx.n_cohorts) if idx.bra_pos[c] == idx.ket_pos[c] and not idx.tr[c] and idx.cohort_size(c)]
     small = min(diag, key=lambda c: idx.bra.sizes[idx.bra_pos[c]])
-    # the widest unit without an S_D block: left sector lb_out, one state of the right sector it meets
-    left, right = ws.left_index.bra, idx.bra
-    widest = max(right.sizes[r] for r in range(len(right.charges)) if r != idx.bra_pos[small])
     eng = E.Engine(0)   # no workspace of an earlier plan
     try:
-        check_sigma(eng, ws, ws.left_index, subset(idx, [small]), "%s L=%d site=%d m=%d" % (model, L, site, m),
-                    min_bytes=8 * widest * max(left.sizes))
+        check_sigma(eng, ws, ws.left_index, subset(idx, [small]), "%s L=%d site=%d m=%d" % (model, L, site, m))
     finally:
         eng.close()
