@@ -332,7 +332,9 @@ int mq_plan_profile(mq_plan* plan, const double* psi, double* sigma, int reps, i
                     double* stage_ms, uint64_t* flops_out, uint64_t* gather_bytes);
 int mq_plan_vector_size(const mq_plan* plan, uint64_t* n_elements);
 int mq_plan_flops(const mq_plan* plan, uint64_t* flops);
-/* Bytes of device workspace held by the plan (T and S buffers and tables). */
+/* Bytes of device memory held by the plan at the time of the call: T and S buffers, tables, W tiles,
+ * and what its applications have allocated so far, each allocation at its full size (buffers from
+ * the context's pools carry up to 25% headroom). */
 int mq_plan_workspace_bytes(const mq_plan* plan, uint64_t* bytes);
 int mq_plan_destroy(mq_plan* plan);
 

@@ -113,6 +113,7 @@ struct DevBuf {
         }
         bytes = n;
     }
+    size_t owned() const { return view ? 0 : bytes; }
     void ensure(size_t n) {
         if (n > bytes) alloc(n);
     }
@@ -502,7 +503,7 @@ struct GemmStage {
             up(d_tile_task, tile_task);
         }
         const uint32_t* table() const { return tile_task.empty() ? nullptr : d_tile_task.as<uint32_t>(); }
-        uint64_t device_bytes() const { return d_tasks.bytes + d_tile_task.bytes; }
+        uint64_t device_bytes() const { return d_tasks.owned() + d_tile_task.owned(); }
     } stream[T_STREAM_N];
     std::vector<int8_t> cls_of;   // per task of `all`: its class, -1 for the tile configurations
     // column-unit tasks run by the wave form of the final stage, numbered for FP64 and for FP32: those
@@ -730,12 +731,13 @@ struct GemmStage {
                                    d_segs.as<GemmSeg>(), tiles[c], b, tb, tt));
         }
     }
+    // of its own allocations (after an autotuning), not of the plan's one table buffer
     uint64_t device_bytes() const {
-        uint64_t n = d_segs.bytes;
-        for (const auto& d : d_tasks) n += d.bytes;
-        for (const auto& d : d_tile_task) n += d.bytes;
+        uint64_t n = d_segs.owned();
+        for (const auto& d : d_tasks) n += d.owned();
+        for (const auto& d : d_tile_task) n += d.owned();
         for (const auto& s : stream) n += s.device_bytes();
-        n += wave64.device_bytes() + wave32.device_bytes();
+        n += wave64.device_bytes() + wave32.device_bytes() + step_final.device_bytes();
         return n;
     }
 };
@@ -775,7 +777,6 @@ struct GatherSet {
         HIPCHK(launch_gather_small(st, d_small.as<GatherRegion>(), uint32_t(small.size()), d_src_off.as<uint64_t>(),
                                    d_alpha.as<double>(), src, dst));
     }
-    uint64_t device_bytes() const { return d_regions.bytes + d_small.bytes + d_src_off.bytes + d_alpha.bytes; }
 };
 
 struct StagePlan {
@@ -3964,8 +3965,13 @@ int mq_plan_workspace_bytes(const mq_plan* p, uint64_t* bytes) {
     return guarded([&] {
         MQ_REQUIRE(p && bytes, "bad argument");
         const StagePlan& P = p->st;
-        *bytes = p->ws.bytes + p->ws32.bytes + p->part.bytes + P.gT.device_bytes() + P.gF.device_bytes() + P.bsr.d_tasks.bytes + P.bsr.d_runs.bytes + P.bsr.d_tile_cols.bytes + P.bsr.d_w64.bytes + P.bsr.d_w32.bytes + P.bsr.d_whi.bytes + P.bsr.d_wlo.bytes + P.red.device_bytes() + P.d_maps.bytes + P.d_units.bytes + P.d_rows.bytes + P.d_regions.bytes +
-                 P.d_small.bytes + P.d_src_off.bytes + P.d_alpha.bytes;
+        // the allocations as they are: the pools' headroom included, the views of one allocation once, and
+        // the tables that the autotuner has replaced by its own
+        uint64_t n = P.tables.bytes + P.wtiles.bytes + P.gT.device_bytes() + P.gF.device_bytes() + P.gU.device_bytes();
+        for (const DevBuf* b : {&p->ws, &p->ws32, &p->part, &p->bf, &p->io, &p->jd_buf, &p->adj_g, &p->d_adj_ptr, &p->d_adj_idx,
+                                &p->d_adj_coef, &p->d_grad})
+            n += b->owned();
+        *bytes = n;
     });
 }
 

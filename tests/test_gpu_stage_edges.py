@@ -69,3 +69,26 @@ def test_right_boundary_with_one_sector(model, L, site, m):
         check_sigma(eng, ws, ws.left_index, subset(idx, [small]), "%s L=%d site=%d m=%d" % (model, L, site, m))
     finally:
         eng.close()
+
+
+def test_workspace_bytes_are_the_plan_s_allocations():
+    """What a second plan of a site takes from the device (the first one's lowering has left its entry
+    staging in the pool) is what it reports, headroom of the pooled buffers included."""
+    ws = SyntheticSite("qc_su2", 16, 7, 256, seed=2)
+    eng = E.Engine(0)
+    try:
+        Lb = E.DeviceBoundary.upload(eng, ws.left_index, ws.random_cohorts(ws.left_index))
+        Rb = E.DeviceBoundary.upload(eng, ws.right_index, ws.random_cohorts(ws.right_index))
+        first = E.SigmaPlan(eng, ws.site_desc, ws.mpo_desc, Lb, Rb)
+        free0 = torch.cuda.mem_get_info()[0]
+        second = E.SigmaPlan(eng, ws.site_desc, ws.mpo_desc, Lb, Rb)
+        taken = free0 - torch.cuda.mem_get_info()[0]
+        print("taken %d reported %d" % (taken, second.workspace_bytes), flush=True)
+        # four allocations (T and S, partial sums, tables, W tiles), each with up to a page of 2 MiB that the
+        # device may have had in reserve
+        assert abs(taken - second.workspace_bytes) <= 4 * (2 << 20)
+        assert first.workspace_bytes == second.workspace_bytes
+        second.close()
+        first.close()
+    finally:
+        eng.close()
