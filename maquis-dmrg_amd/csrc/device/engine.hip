@@ -3445,6 +3445,18 @@ void lower_sigma_grouped(mq_plan* p, const SiteLayout& site, const Mpo& W, uint6
 
 extern "C" {
 
+// The adjoint's products T_g^T U_g have at most a few tens of tiles each: from 6.5e6 flops a group on average
+// they run side by side on the side streams.  SU2U1, one after another / side by side: L=16 m=256 (1.1e8 a
+// group) 3.45 / 2.37 ms, L=12 m=100 (8.6e6) 1.02 / 0.84, L=14 m=60 (4.6e6) 0.81 / 0.91, L=10 m=67 (2.8e6)
+// 0.59 / 0.66: below it the launches bound both, and those to several streams cost more.
+static double group_flops(const StagePlan::LibGemm& g) { return 2.0 * g.M * g.N * g.K; }
+static bool adjoint_forks(const StagePlan& P) {
+    constexpr double FORK_FLOPS = 6.5e6;
+    double total = 0;
+    for (const auto& g : P.lib) total += group_flops(g);
+    return total > 0 && total >= FORK_FLOPS * double(P.lib.size());
+}
+
 // The context's side streams, their events and library handles, created at their first use.
 static void side_streams(mq_ctx* ctx) {
     if (!ctx->side.empty()) return;
@@ -3453,8 +3465,6 @@ static void side_streams(mq_ctx* ctx) {
     for (int k = 0; k < mq_ctx::NSIDE; ++k) {
         HIPCHK(hipStreamCreateWithFlags(&ctx->side[k], hipStreamNonBlocking));
         HIPCHK(hipEventCreateWithFlags(&ctx->side_ev[k], hipEventDisableTiming));
-        ctx->lt_ws_side.push_back(std::make_unique<DevBuf>());
-        ctx->lt_ws_side.back()->alloc(LT_WORKSPACE);
         rocblas_handle h = nullptr;
         BLASCHK(rocblas_create_handle(&h));
         ctx->side_blas.push_back(h);
@@ -3515,7 +3525,6 @@ int mq_sigma_plan_create_ex(mq_ctx* ctx, const mq_site_desc* site, const mq_mpo_
         }
         const bool adjoint = (algorithm & MQ_SIGMA_ADJOINT) != 0;
         algorithm &= ~int(MQ_SIGMA_ADJOINT);
-        if (adjoint) side_streams(ctx);   // mq_sigma_adjoint's products
         MQ_REQUIRE(algorithm == MQ_SIGMA_GROUPED,
                    adjoint ? "the sigma adjoint needs a GROUPED plan" : "unknown sigma algorithm");
         Mpo W(*mpo);
@@ -3528,6 +3537,7 @@ int mq_sigma_plan_create_ex(mq_ctx* ctx, const mq_site_desc* site, const mq_mpo_
         lower_sigma_grouped(p.get(), L, W, wd_elems, ws_init_off, adjoint);
         trace_phase("lower: final stage");
         StagePlan& P = p->st;
+        if (adjoint && adjoint_forks(P)) side_streams(ctx);
         P.blas = ctx->blas;
         P.lt_ctx = ctx;
         P.finish_tables();
@@ -3641,6 +3651,13 @@ int mq_sigma_apply_batched(mq_ctx* ctx, int n, mq_plan* const* plans, const doub
         hipStream_t st = ctx->stream;
         constexpr int NSIDE = mq_ctx::NSIDE;
         side_streams(ctx);
+        // hipBLASLt runs the reduced-precision S stage of MQ_S_DENSE=1 plans alone
+        if (precision != MQ_PREC_F64 && std::any_of(plans, plans + n, [](const mq_plan* p) { return !p->st.bsr_on; }))
+            while (ctx->lt_ws_side.size() < size_t(NSIDE)) {
+                auto b = std::make_unique<DevBuf>();
+                b->alloc(LT_WORKSPACE);
+                ctx->lt_ws_side.push_back(std::move(b));
+            }
         // operand slots and workspaces of every plan exist before any capture
         std::vector<Bases> bs(n);
         std::vector<double*> ins(n), outs(n);
@@ -3823,24 +3840,18 @@ int mq_sigma_adjoint(mq_plan* p, const double* psi, double* grad) {
         P.stage(1, st, b, MODE_F64);
         HIPCHK(launch_fill(st, ws + p->s_region0, p->s_region1 - p->s_region0, 0.0));
         P.run_u(st, b);
-        // G_g = T_g^T U_g in the W_D layout: the derivative of psi . sigma with respect to W_D.  A group's
-        // product has at most a few tens of tiles: from 6.5e6 flops a group on average the groups run side by
-        // side on the side streams, each next one (largest first) on the stream with the least work.  SU2U1,
-        // one after another / side by side: L=16 m=256 (1.1e8 a group) 3.45 / 2.37 ms, L=12 m=100 (8.6e6)
-        // 1.02 / 0.84, L=14 m=60 (4.6e6) 0.81 / 0.91, L=10 m=67 (2.8e6) 0.59 / 0.66: below it the launches
-        // bound both, and those to several streams cost more.
-        constexpr double FORK_FLOPS = 6.5e6;
+        // G_g = T_g^T U_g in the W_D layout: the derivative of psi . sigma with respect to W_D.  Where it pays
+        // (adjoint_forks) the groups run side by side on the side streams, each next one (largest first) on
+        // the stream with the least work.
         const double one = 1.0, zero = 0.0;
         double* G = p->adj_g.as<double>();
-        auto work = [&](size_t i) { return 2.0 * P.lib[i].M * P.lib[i].N * P.lib[i].K; };
+        auto work = [&](size_t i) { return group_flops(P.lib[i]); };
         auto product = [&](rocblas_handle h, size_t i) {
             const auto& g = P.lib[i];
             BLASCHK(rocblas_dgemm(h, rocblas_operation_transpose, rocblas_operation_none, g.K, g.N, g.M, &one, ws + g.a_off,
                                   g.lda, ws + g.c_off, g.ldc, &zero, G + (g.b_off - p->ws_init_off), g.K));
         };
-        double total = 0;
-        for (size_t i = 0; i < P.lib.size(); ++i) total += work(i);
-        if (total < FORK_FLOPS * double(P.lib.size())) {
+        if (!adjoint_forks(P)) {
             BLASCHK(rocblas_set_stream(P.blas, st));
             for (size_t i = 0; i < P.lib.size(); ++i) product(P.blas, i);
         } else {

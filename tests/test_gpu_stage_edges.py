@@ -92,3 +92,24 @@ def test_workspace_bytes_are_the_plan_s_allocations():
         first.close()
     finally:
         eng.close()
+
+
+def test_adjoint_plan_takes_no_memory_it_does_not_use():
+    """An adjoint plan of groups too small to run side by side takes no side streams (their library
+    handles hold device memory), and no adjoint plan takes hipBLASLt workspaces (64 MiB a stream)."""
+    ws = SyntheticSite("qc_su2", 10, 4, 67, seed=2)
+    eng = E.Engine(0)
+    try:
+        Lb = E.DeviceBoundary.upload(eng, ws.left_index, ws.random_cohorts(ws.left_index))
+        Rb = E.DeviceBoundary.upload(eng, ws.right_index, ws.random_cohorts(ws.right_index))
+        psi = torch.from_numpy(ws.random_psi()).to("cuda:0")
+        torch.cuda.synchronize()
+        free0 = torch.cuda.mem_get_info()[0]
+        plan = E.SigmaPlan(eng, ws.site_desc, ws.mpo_desc, Lb, Rb, algorithm=E.SIGMA_GROUPED, adjoint=True)
+        taken = free0 - torch.cuda.mem_get_info()[0]
+        print("taken %d reported %d" % (taken, plan.workspace_bytes), flush=True)
+        assert taken - plan.workspace_bytes < 64 << 20
+        assert np.all(np.isfinite(plan.adjoint(psi)))
+        plan.close()
+    finally:
+        eng.close()
