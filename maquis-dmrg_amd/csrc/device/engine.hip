@@ -375,6 +375,16 @@ struct mq_ctx {
         return blas;
     }
     hipEvent_t fork_ev = nullptr;
+    void drop_side() {
+        for (auto h : side_blas) (void)rocblas_destroy_handle(h);
+        for (auto sd : side) (void)hipStreamDestroy(sd);
+        for (auto e : side_ev) (void)hipEventDestroy(e);
+        if (fork_ev) (void)hipEventDestroy(fork_ev);
+        side_blas.clear();
+        side.clear();
+        side_ev.clear();
+        fork_ev = nullptr;
+    }
     std::map<std::pair<std::vector<const mq_plan*>, int>, BatchGraph> batches;
     // autotuned tile policies, keyed by (stage, precision, grouped, log2 flop histogram over size classes)
     std::map<std::vector<int>, std::array<int, 5>> tuned;
@@ -1677,10 +1687,7 @@ int mq_ctx_destroy(mq_ctx* ctx) {
         if (!ctx) return;
         (void)hipStreamSynchronize(ctx->stream);
         ctx->drop_batches();
-        for (auto h : ctx->side_blas) (void)rocblas_destroy_handle(h);
-        for (auto sd : ctx->side) (void)hipStreamDestroy(sd);
-        for (auto e : ctx->side_ev) (void)hipEventDestroy(e);
-        if (ctx->fork_ev) (void)hipEventDestroy(ctx->fork_ev);
+        ctx->drop_side();
         ctx->pool_clear();
         if (ctx->wd_host) (void)hipHostFree(ctx->wd_host);
         if (ctx->tab_host) (void)hipHostFree(ctx->tab_host);
@@ -3457,20 +3464,29 @@ static bool adjoint_forks(const StagePlan& P) {
     return total > 0 && total >= FORK_FLOPS * double(P.lib.size());
 }
 
-// The context's side streams, their events and library handles, created at their first use.
+// The context's side streams, their events and library handles, created at their first use: all of them, or
+// none when one cannot be made.
 static void side_streams(mq_ctx* ctx) {
     if (!ctx->side.empty()) return;
-    ctx->side.resize(mq_ctx::NSIDE);
-    ctx->side_ev.resize(mq_ctx::NSIDE);
-    for (int k = 0; k < mq_ctx::NSIDE; ++k) {
-        HIPCHK(hipStreamCreateWithFlags(&ctx->side[k], hipStreamNonBlocking));
-        HIPCHK(hipEventCreateWithFlags(&ctx->side_ev[k], hipEventDisableTiming));
-        rocblas_handle h = nullptr;
-        BLASCHK(rocblas_create_handle(&h));
-        ctx->side_blas.push_back(h);
-        BLASCHK(rocblas_set_stream(h, ctx->side[k]));
+    try {
+        HIPCHK(hipEventCreateWithFlags(&ctx->fork_ev, hipEventDisableTiming));
+        for (int k = 0; k < mq_ctx::NSIDE; ++k) {
+            hipStream_t sd = nullptr;
+            HIPCHK(hipStreamCreateWithFlags(&sd, hipStreamNonBlocking));
+            ctx->side.push_back(sd);
+            hipEvent_t ev = nullptr;
+            HIPCHK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+            ctx->side_ev.push_back(ev);
+            rocblas_handle h = nullptr;
+            BLASCHK(rocblas_create_handle(&h));
+            ctx->side_blas.push_back(h);
+            BLASCHK(rocblas_set_stream(h, sd));
+        }
+    } catch (...) {
+        (void)hipGetLastError();
+        ctx->drop_side();
+        throw;
     }
-    HIPCHK(hipEventCreateWithFlags(&ctx->fork_ev, hipEventDisableTiming));
 }
 
 int mq_sigma_plan_create_from_schedule(mq_ctx* ctx, const mq_schedule_desc* sched, uint32_t n_ket_blocks,
@@ -3537,7 +3553,6 @@ int mq_sigma_plan_create_ex(mq_ctx* ctx, const mq_site_desc* site, const mq_mpo_
         lower_sigma_grouped(p.get(), L, W, wd_elems, ws_init_off, adjoint);
         trace_phase("lower: final stage");
         StagePlan& P = p->st;
-        if (adjoint && adjoint_forks(P)) side_streams(ctx);
         P.blas = ctx->blas;
         P.lt_ctx = ctx;
         P.finish_tables();
@@ -3561,6 +3576,12 @@ int mq_sigma_plan_create_ex(mq_ctx* ctx, const mq_site_desc* site, const mq_mpo_
         P.upload_all(ctx);
         HIPCHK(hipStreamSynchronize(ctx->stream));
         trace_phase("plan: upload");
+        if (adjoint && adjoint_forks(P)) {
+            try {
+                side_streams(ctx);
+            } catch (const Error&) {   // no room left for their handles: the products run on one stream
+            }
+        }
         p->grouped = true;
         p->ws_init_elems = wd_elems;
         p->ws_init_off = ws_init_off;
@@ -3825,12 +3846,22 @@ int mq_sigma_adjoint(mq_plan* p, const double* psi, double* grad) {
         mq_ctx* ctx = p->ctx;
         hipStream_t st = ctx->stream;
         StagePlan& P = p->st;
-        if (!p->d_grad.p) {
-            upload(p->d_adj_ptr, p->adj_ptr, st);
-            upload(p->d_adj_idx, p->adj_idx, st);
-            upload(p->d_adj_coef, p->adj_coef, st);
-            p->d_grad.alloc(std::max<uint32_t>(p->n_terms, 1) * sizeof(double));
-            p->adj_g.alloc_zeroed(std::max<uint64_t>(P.ws_elems - p->ws_init_off, 1) * sizeof(double), st);
+        if (!p->adj_g.p) {
+            auto buffers = [&] {
+                upload(p->d_adj_ptr, p->adj_ptr, st);
+                upload(p->d_adj_idx, p->adj_idx, st);
+                upload(p->d_adj_coef, p->adj_coef, st);
+                p->d_grad.alloc(std::max<uint32_t>(p->n_terms, 1) * sizeof(double));
+                p->adj_g.alloc_zeroed(std::max<uint64_t>(P.ws_elems - p->ws_init_off, 1) * sizeof(double), st);
+            };
+            try {
+                buffers();
+            } catch (const Error& e) {   // the side streams' handles make room: the products run on one stream
+                if (e.code != MQ_ERR_NOMEM || ctx->side.empty()) throw;
+                HIPCHK(hipStreamSynchronize(st));
+                ctx->drop_side();
+                buffers();
+            }
         }
         Bases b = p->bases(psi, nullptr, MODE_F64);
         double* ws = b.p[BASE_WS];
@@ -3851,7 +3882,7 @@ int mq_sigma_adjoint(mq_plan* p, const double* psi, double* grad) {
             BLASCHK(rocblas_dgemm(h, rocblas_operation_transpose, rocblas_operation_none, g.K, g.N, g.M, &one, ws + g.a_off,
                                   g.lda, ws + g.c_off, g.ldc, &zero, G + (g.b_off - p->ws_init_off), g.K));
         };
-        if (!adjoint_forks(P)) {
+        if (ctx->side.empty() || !adjoint_forks(P)) {
             BLASCHK(rocblas_set_stream(P.blas, st));
             for (size_t i = 0; i < P.lib.size(); ++i) product(P.blas, i);
         } else {
