@@ -564,11 +564,16 @@ struct GemmStage {
             if (g.K <= T_STREAM_KMAX[c]) return c;
         return -1;
     }
-    // Flops per size class: the block-size histogram the autotuner's decisions are keyed on.
-    std::vector<uint64_t> class_flops(const std::vector<GemmSeg>& segs) const {
+    // Flops per size class of the tasks whose launch in `mode` follows the tile policy (the streamed and
+    // wave kernels have tiles of their own): the block-size histogram the autotuner's decisions are keyed on.
+    std::vector<uint64_t> class_flops(const std::vector<GemmSeg>& segs, int mode) const {
         std::vector<uint64_t> f(N_SIZE_CLASS, 0);
-        for (const auto& t : all)
+        if (mode == MODE_F64 && wave64_all) return f;
+        for (size_t i = 0; i < all.size(); ++i) {
+            const GemmTask& t = all[i];
+            if (cls_of[i] >= 0) continue;
             for (uint32_t s = t.seg0; s < t.seg1; ++s) f[size_class(t.M)] += 2ull * t.M * t.N * segs[s].K;
+        }
         return f;
     }
     // streamed: take the streamed T kernel for the tasks it suits (plans whose T stage writes T_D in its
@@ -3782,7 +3787,8 @@ int mq_plan_autotune(mq_plan* p, int precision, int* timed) {
         for (StageRef sr : {StageRef{1, &P.gT, &P.t_segs}, StageRef{3, &P.gF, &P.f_segs}}) {
             if (library_only) break;
             GemmStage& G = *sr.g;
-            std::vector<uint64_t> cf = G.class_flops(*sr.segs);
+            std::vector<uint64_t> cf = G.class_flops(*sr.segs, precision);
+            if (std::all_of(cf.begin(), cf.end(), [](uint64_t f) { return f == 0; })) continue;   // nothing to tune
             std::vector<int> key = {sr.k, precision, int(p->grouped)};
             for (auto f : cf) key.push_back(f ? int(std::log2(double(f))) : -1);
             auto apply = [&](const TilePolicy& pol) {

@@ -1,6 +1,10 @@
 """Forms of the stage kernels and of the plans around them that the chains' ordinary sites do not
 reach: boundaries with cohorts left out, sectors beyond one tile of the step kernel, the adjoint's
 products side by side, wide groups, large stages."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 import torch
@@ -144,3 +148,33 @@ def test_adjoint_without_room_for_side_streams():
     want = gradient()
     # the plan and the adjoint's buffers take about 90 MiB, the four library handles about 150 MiB each
     assert np.array_equal(gradient(room=400 << 20), want)
+
+
+AUTOTUNE = """
+import numpy as np
+from mqdmrg import engine as E
+from mqdmrg.workloads import SyntheticSite
+ws = SyntheticSite("heisenberg", 16, 7, 150, seed=3)
+eng = E.Engine(0)
+Lb = E.DeviceBoundary.upload(eng, ws.left_index, ws.random_cohorts(ws.left_index))
+Rb = E.DeviceBoundary.upload(eng, ws.right_index, ws.random_cohorts(ws.right_index))
+plan = E.SigmaPlan(eng, ws.site_desc, ws.mpo_desc, Lb, Rb)
+print("timed", plan.autotune(E.PREC_F64), plan.autotune(E.PREC_F32))
+plan.close()
+eng.close()
+"""
+
+
+def test_autotune_times_only_what_a_choice_changes():
+    """A small stage's final tasks run in the wave kernel in FP64 whatever tile is chosen for them: their
+    tiles are not timed there (and noise picks none, which FP32 applications of the plan would then use).
+    MQ_F_GENERIC=1 sends them to the tile kernels, where every candidate is timed."""
+    def timed(**env):
+        r = subprocess.run([sys.executable, "-c", AUTOTUNE], capture_output=True, text=True, timeout=100,
+                           env=dict(os.environ, PYTHONPATH=os.pathsep.join(sys.path), **env))
+        assert r.returncode == 0, r.stderr[-2000:]
+        return [int(x) for x in r.stdout.split("timed")[1].split()]
+
+    wave, tiles = timed(), timed(MQ_F_GENERIC="1")
+    print("timed FP64, FP32: wave kernel %s, tile kernels %s" % (wave, tiles), flush=True)
+    assert 0 < wave[0] < tiles[0]
