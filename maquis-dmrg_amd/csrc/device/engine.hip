@@ -582,8 +582,9 @@ struct GemmStage {
     void build(const std::vector<GemmTask>& tasks, const std::vector<GemmSeg>& segs, const std::vector<GemmRow>& rows,
                const std::vector<uint32_t>& maps, bool streamed, bool f64_only) {
         static const bool generic = std::getenv("MQ_T_GENERIC") != nullptr;
+        static const bool generic_f = std::getenv("MQ_F_GENERIC") != nullptr;
         all = tasks;
-        if (f64_only && !generic) {
+        if (f64_only && !generic_f) {
             bool every = !all.empty();
             for (const auto& t : all) every = every && step_task(t, segs, rows, maps);
             if (every) {
@@ -595,7 +596,6 @@ struct GemmStage {
         cls_of.assign(all.size(), -1);
         if (streamed && !generic)
             for (size_t i = 0; i < all.size(); ++i) cls_of[i] = int8_t(stream_class(all[i], segs));
-        static const bool generic_f = std::getenv("MQ_F_GENERIC") != nullptr;
         if (!generic_f) {
             // FP64: a stage whose 64 x 64 tiles would leave CUs idle runs in the wave form altogether
             // (its chains split over 4 waves)

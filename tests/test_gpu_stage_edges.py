@@ -178,3 +178,39 @@ def test_autotune_times_only_what_a_choice_changes():
     wave, tiles = timed(), timed(MQ_F_GENERIC="1")
     print("timed FP64, FP32: wave kernel %s, tile kernels %s" % (wave, tiles), flush=True)
     assert 0 < wave[0] < tiles[0]
+
+
+STEP = """
+import hashlib
+import sys
+import numpy as np
+import torch
+from mqdmrg import engine as E, mps
+from mqdmrg.symmetry import SiteLayout
+from mqdmrg.workloads import SyntheticSite
+ws = SyntheticSite("qc_su2", 10, 4, 131, seed=3)
+k = ws.site + 1
+lay = SiteLayout(ws.bonds[k], ws.basis.phys, ws.bonds[k + 1])
+sd, md = E.SiteDesc(ws.basis.sym, ws.bonds[k], ws.basis.phys, ws.bonds[k + 1]), E.MpoDesc(ws.mpo[k])
+eng = E.Engine(0)
+b = E.DeviceBoundary.upload(eng, ws.right_index, ws.random_cohorts(ws.right_index))
+bra, ket = (torch.from_numpy(mps.random_site_vector(lay, ws.rng)).to("cuda:0") for _ in range(2))
+h = hashlib.sha256()
+for x in E.right_step(eng, sd, md, bra, ket, b).download():
+    h.update(np.ascontiguousarray(x).tobytes())
+print("digest", h.hexdigest())
+"""
+
+
+def test_generic_switches_are_of_one_stage_each():
+    """MQ_T_GENERIC is the T stage's switch and MQ_F_GENERIC the final stage's, of a boundary step too: the
+    final stage's own kernel and the generic one sum in another order, so turning it off shows in the bits
+    with either form of the T stage."""
+    def digest(**env):
+        r = subprocess.run([sys.executable, "-c", STEP], capture_output=True, text=True, timeout=100,
+                           env=dict(os.environ, PYTHONPATH=os.pathsep.join(sys.path), **env))
+        assert r.returncode == 0, r.stderr[-2000:]
+        return r.stdout.split("digest")[1].strip()
+
+    assert digest() != digest(MQ_F_GENERIC="1")
+    assert digest(MQ_T_GENERIC="1") != digest(MQ_T_GENERIC="1", MQ_F_GENERIC="1")
