@@ -73,6 +73,21 @@ __device__ inline void split2(float x0, float x1, uint32_t& hi, uint32_t& lo) {
                                           (__bf16)(x1 - __uint_as_float(hi & 0xffff0000u))});
 }
 
+// The same of two elements of B, held in FP64, by one rule for both kernels: hi is the bf16 nearest to the
+// FP32 value, in the first 16-key step nearest to the FP64 value; lo = bf16(FP32 value - hi).  The two differ
+// where the FP32 value lies halfway between two bf16 and the FP64 value does not; hi + lo is the FP32 value
+// to the same 17 bits either way.  The empty asm hides where the FP32 values come from: a conversion of them
+// to bf16 would otherwise be made from the FP64 values wherever the compiler sees those.
+template <bool FIRST>
+__device__ inline void split_b(double d0, double d1, uint32_t& hi, uint32_t& lo) {
+    float x0 = float(d0), x1 = float(d1);
+    asm("" : "+v"(x0), "+v"(x1));
+    hi = FIRST ? __builtin_bit_cast(uint32_t, bf2{(__bf16)d0, (__bf16)d1})
+               : __builtin_bit_cast(uint32_t, bf2{(__bf16)x0, (__bf16)x1});
+    lo = __builtin_bit_cast(uint32_t, bf2{(__bf16)(x0 - __uint_as_float(hi << 16)),
+                                          (__bf16)(x1 - __uint_as_float(hi & 0xffff0000u))});
+}
+
 __device__ inline uint32_t task_of(const GemmTask* tasks, uint32_t n_tasks, const uint32_t* tile_task, uint32_t tile) {
     if (tile_task) return tile_task[tile];
     if (n_tasks == gridDim.x) return tile;
@@ -166,7 +181,7 @@ void t_stack_kernel(const GemmTask* __restrict__ tasks, uint32_t n_tasks, const 
             }
         }
     };
-    auto lstore = [&](int buf, uint32_t k0) {
+    auto lstore = [&](int buf, uint32_t k0, auto first) {
         TsSmem<MODE, BM>& s = sm[buf];
         T xa[KPT], xb[KPT];
 #pragma unroll
@@ -180,7 +195,7 @@ void t_stack_kernel(const GemmTask* __restrict__ tasks, uint32_t n_tasks, const 
 #pragma unroll
             for (int e = 0; e < KPT / 2; ++e) {
                 split2(xa[2 * e], xa[2 * e + 1], ah[e], al[e]);
-                split2(xb[2 * e], xb[2 * e + 1], bh[e], bl[e]);
+                split_b<decltype(first)::value>(vb[2 * e], vb[2 * e + 1], bh[e], bl[e]);
             }
             if constexpr (KPT == 8) {
                 *reinterpret_cast<uint4*>(&s.ahi[a_m][a_k]) = uint4{ah[0], ah[1], ah[2], ah[3]};
@@ -265,7 +280,7 @@ void t_stack_kernel(const GemmTask* __restrict__ tasks, uint32_t n_tasks, const 
     if (K > 0) {
         uint32_t k0 = 0;
         gload(k0);
-        lstore(0, k0);
+        lstore(0, k0, std::true_type{});
         __syncthreads();
         int buf = 0;
         while (true) {
@@ -274,7 +289,7 @@ void t_stack_kernel(const GemmTask* __restrict__ tasks, uint32_t n_tasks, const 
             if (more) gload(k1);
             compute(buf);
             if (!more) break;
-            lstore(buf ^ 1, k1);
+            lstore(buf ^ 1, k1, std::false_type{});
             __syncthreads();
             buf ^= 1;
             k0 = k1;
@@ -486,19 +501,8 @@ void t_stream_kernel(const GemmTask* __restrict__ tasks, uint32_t n_tasks, const
                 }
             }
         };
-        // BF16X3: bf16 hi / lo of two elements of B.  t_stack_kernel's compiled form rounds the first step's
-        // hi from the FP64 value and the others' from its FP32 rounding; so does this.  They differ only
-        // where the FP32 value lies halfway between two bf16 (tie), so the longer conversion runs only
-        // for a first step that holds one (one in a hundred).
-        auto split = [&](double dx, double dy, auto first, uint32_t& h, uint32_t& l) {
-            const float x = float(dx), y = float(dy);
-            if constexpr (decltype(first)::value)
-                h = __builtin_bit_cast(uint32_t, bf2{(__bf16)dx, (__bf16)dy});
-            else   // (a C++ conversion of x would be folded into one of dx)
-                asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(h) : "v"(x), "v"(y));
-            l = __builtin_bit_cast(uint32_t, bf2{(__bf16)(x - __uint_as_float(h << 16)),
-                                                 (__bf16)(y - __uint_as_float(h & 0xffff0000u))});
-        };
+        // BF16X3: the first step's split differs only where an FP32 value lies halfway between two bf16, so its
+        // longer conversion runs only for a first step that holds one (one in a hundred)
         auto put = [&](auto first) {   // the loaded step into the wave's LDS, in the arithmetic's type
 #pragma unroll
             for (int v = 0; v < NV; ++v) {
@@ -507,7 +511,7 @@ void t_stream_kernel(const GemmTask* __restrict__ tasks, uint32_t n_tasks, const
                     const int k = b_k + (128 / WC) * v;
                     if constexpr (BF) {
                         uint32_t h, l;
-                        split(vb[v][0], vb[v][1], first, h, l);
+                        split_b<decltype(first)::value>(vb[v][0], vb[v][1], h, l);
                         wb[0][b_n][k] = uint16_t(h);
                         wb[0][b_n + 1][k] = uint16_t(h >> 16);
                         wb[1][b_n][k] = uint16_t(l);
@@ -520,7 +524,7 @@ void t_stream_kernel(const GemmTask* __restrict__ tasks, uint32_t n_tasks, const
                     const int n = b_n + 8 * v;
                     if constexpr (BF) {
                         uint32_t h, l;
-                        split(vb[v][0], vb[v][1], first, h, l);
+                        split_b<decltype(first)::value>(vb[v][0], vb[v][1], h, l);
                         *reinterpret_cast<uint32_t*>(&wb[0][n][b_k]) = h;
                         *reinterpret_cast<uint32_t*>(&wb[1][n][b_k]) = l;
                     } else {

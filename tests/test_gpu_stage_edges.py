@@ -214,3 +214,30 @@ def test_generic_switches_are_of_one_stage_each():
 
     assert digest() != digest(MQ_F_GENERIC="1")
     assert digest(MQ_T_GENERIC="1") != digest(MQ_T_GENERIC="1", MQ_F_GENERIC="1")
+
+
+@pytest.mark.parametrize("model,L,site,m", [("heisenberg", 20, 9, 420), ("qc_su2", 10, 4, 131), ("qc", 10, 4, 150),
+                                            ("heisenberg", 24, 11, 1100)])
+def test_bf16x3_of_halfway_values(eng, model, L, site, m):
+    """BF16x3 where every value of the right boundary is, rounded to FP32, halfway between two bf16 and in
+    FP64 a little above or below: the case in which the T stage's split depends on what it rounds.  The
+    split keeps 17 bits whichever way such a value goes."""
+    ws = SyntheticSite(model, L, site, m, seed=L + m)
+    Lc = ws.random_cohorts(ws.left_index)
+
+    def halfway(x):
+        bits = (x.astype(np.float32).view(np.uint32) & 0xffff0000) | 0x8000
+        return bits.view(np.float32).astype(np.float64) * (1 + 1e-9 * np.sign(ws.rng.standard_normal(len(x))))
+    Rc = [halfway(x) if x is not None else None for x in ws.random_cohorts(ws.right_index)]
+    psi_h = ws.random_psi()
+    ref = O.SigmaOracle(ws.site_desc, ws.mpo_desc, host_boundary(ws.left_index, Lc), host_boundary(ws.right_index, Rc)).apply(psi_h)
+    Lb, Rb = E.DeviceBoundary.upload(eng, ws.left_index, Lc), E.DeviceBoundary.upload(eng, ws.right_index, Rc)
+    plan = E.SigmaPlan(eng, ws.site_desc, ws.mpo_desc, Lb, Rb)
+    psi = torch.from_numpy(psi_h).to("cuda:0")
+    out = torch.full_like(psi, float("nan"))
+    plan.apply(psi, out, precision=E.PREC_BF16X3)
+    eng.sync()
+    err = np.linalg.norm(out.cpu().numpy() - ref) / np.linalg.norm(ref)
+    print("%s L=%d site=%d m=%d: %.2e" % (model, L, site, m, err), flush=True)
+    assert err <= RTOL[E.PREC_BF16X3]
+    plan.close()
