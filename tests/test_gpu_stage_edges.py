@@ -241,3 +241,131 @@ def test_bf16x3_of_halfway_values(eng, model, L, site, m):
     print("%s L=%d site=%d m=%d: %.2e" % (model, L, site, m, err), flush=True)
     assert err <= RTOL[E.PREC_BF16X3]
     plan.close()
+
+
+SIGMA_SHAPES = [("heisenberg", 16, 7, 150), ("heisenberg", 12, 1, 64), ("hubbard", 12, 5, 301), ("hubbard", 10, 7, 90),
+                ("qc", 8, 3, 77), ("qc", 10, 1, 60), ("qc_su2", 10, 4, 131), ("qc_su2", 12, 8, 57), ("qc_su2", 14, 6, 101),
+                ("heisenberg", 20, 9, 420), ("heisenberg", 24, 11, 1100)]
+
+
+@pytest.mark.parametrize("model,L,site,m", SIGMA_SHAPES)
+def test_every_output_block_matches_oracle(eng, model, L, site, m):
+    """sigma block by block and in strips of 64 columns: a wrong edge tile of a small block does not drown
+    in the norm of the whole vector.  An element's error is measured against the larger of its strip's rms
+    and the vector's.  BF16x3 keeps 17 bits of every operand (7.6e-6); a lost low part would be 1.5e-3 in
+    the elements it concerns."""
+    ws = SyntheticSite(model, L, site, m, seed=L + m)
+    Lc, Rc = ws.random_cohorts(ws.left_index), ws.random_cohorts(ws.right_index)
+    psi_h = ws.random_psi()
+    ref = O.SigmaOracle(ws.site_desc, ws.mpo_desc, host_boundary(ws.left_index, Lc), host_boundary(ws.right_index, Rc)).apply(psi_h)
+    Lb, Rb = E.DeviceBoundary.upload(eng, ws.left_index, Lc), E.DeviceBoundary.upload(eng, ws.right_index, Rc)
+    plan = E.SigmaPlan(eng, ws.site_desc, ws.mpo_desc, Lb, Rb)
+    psi = torch.from_numpy(psi_h).to("cuda:0")
+    lay = ws.layout
+    n = sum(ls * cols for ls, cols in zip(lay.left.sizes, lay.rp_cols))
+    rms = np.linalg.norm(ref) / np.sqrt(n)
+    for prec, tol in RTOL.items():
+        out = torch.full_like(psi, float("nan"))
+        plan.apply(psi, out, precision=prec)
+        eng.sync()
+        got, worst = out.cpu().numpy(), 0.0
+        for ls, cols, o in zip(lay.left.sizes, lay.rp_cols, lay.rp_offset):
+            for c in range(0, cols, 64):
+                a, b = o + c * ls, o + min(c + 64, cols) * ls
+                scale = max(np.linalg.norm(ref[a:b]), rms * np.sqrt(b - a))
+                worst = max(worst, np.linalg.norm(got[a:b] - ref[a:b]) / scale)
+        print("%s L=%d site=%d m=%d precision %d: worst strip %.2e" % (model, L, site, m, prec, worst), flush=True)
+        assert worst <= tol
+    plan.close()
+
+
+def final_tiles(ws, cols, small_only):
+    """Tiles of 32 rows x `cols` columns of the final stage's tasks (one per output block and part of its
+    summation range, of about 2048 keys each), all of them or those of at most 32 rows."""
+    idx, lay, n = ws.left_index, ws.layout, 0
+    blocks = {(int(idx.bra_pos[c]), int(idx.ket_pos[c])): int((idx.offsets[c] > -1).sum()) for c in range(idx.n_cohorts)}
+    for lo, (ls, N) in enumerate(zip(lay.left.sizes, lay.rp_cols)):
+        segs = []
+        for lb, s in enumerate(lay.left.sizes):
+            per = max(1, 2048 // s)
+            segs += [min(per, blocks.get((lo, lb), 0) - j) * s for j in range(0, blocks.get((lo, lb), 0), per)]
+        if N and segs and (ls <= 32 or not small_only):
+            n += min(len(segs), 64, -(-sum(segs) // 2048)) * (-(-ls // 32)) * (-(-N // cols))
+    return n
+
+
+@pytest.mark.parametrize("m", [500, 1200])
+def test_wave_form_of_32_rows(eng, m):
+    """Stages with at least 1024 tiles of the final stage's wave form, which then takes 32 rows per wave:
+    in FP64 (m = 500, 1200) and in FP32 (m = 1200)."""
+    ws = SyntheticSite("qc", 12 if m == 500 else 16, 5 if m == 500 else 7, m, seed=m)
+    assert final_tiles(ws, 16, m == 1200) >= 1024
+    assert m == 500 or final_tiles(ws, 64, True) >= 1024
+    check_sigma(eng, ws, ws.left_index, ws.right_index, "qc m=%d" % m)
+
+
+@pytest.mark.parametrize("kind", ["left", "right"])
+@pytest.mark.parametrize("model,L,site,m", [("heisenberg", 20, 9, 420), ("heisenberg", 24, 11, 1100), ("qc_su2", 14, 6, 1500)])
+def test_steps_over_sectors_of_several_tiles(eng, kind, model, L, site, m):
+    """Boundary steps whose tasks have several column tiles (a sector of the bra above 64, with a remainder)
+    and several row tiles per block."""
+    from mqdmrg import mps
+    from mqdmrg.symmetry import SiteLayout
+    ws = SyntheticSite(model, L, site, m, seed=L + m)
+    k = site if kind == "left" else site + 1
+    index = ws.left_index if kind == "left" else ws.right_index
+    lay = SiteLayout(ws.bonds[k], ws.basis.phys, ws.bonds[k + 1])
+    # the new boundary's sectors: its tasks' columns
+    sectors = (lay.right if kind == "left" else lay.left).sizes
+    assert max(sectors) > 64 and any(s > 64 and s % 64 and s % 16 for s in sectors)
+    sd, md = E.SiteDesc(ws.basis.sym, ws.bonds[k], ws.basis.phys, ws.bonds[k + 1]), E.MpoDesc(ws.mpo[k])
+    coh = ws.random_cohorts(index)
+    hb = host_boundary(index, coh)
+    bra, ket = mps.random_site_vector(lay, ws.rng), mps.random_site_vector(lay, ws.rng)
+    d = lambda x: torch.from_numpy(np.ascontiguousarray(x)).to("cuda:0")  # noqa: E731
+    b = E.DeviceBoundary.upload(eng, index, coh)
+    if kind == "left":
+        ref = O.left_step(sd, md, mps.rp_to_lp(lay, bra), ket, hb, True)
+        new = E.left_step(eng, sd, md, d(mps.rp_to_lp(lay, bra)), d(ket), b)
+    else:
+        ref = O.right_step(sd, md, bra, ket, hb, True)
+        new = E.right_step(eng, sd, md, d(bra), d(ket), b)
+    got = new.download()
+    rms = np.sqrt(sum(float(np.sum(y ** 2)) for y in ref.cohorts) / max(1, sum(len(y) for y in ref.cohorts)))
+    worst = 0.0
+    for x, y in zip(got, ref.cohorts):
+        if len(y):
+            worst = max(worst, np.linalg.norm(x - y) / max(np.linalg.norm(y), rms * np.sqrt(len(y))))
+    print("%s %s L=%d site=%d m=%d: worst cohort %.2e" % (kind, model, L, site, m, worst), flush=True)
+    assert worst <= RTOL[E.PREC_F64]
+
+
+@pytest.mark.parametrize("model,L,site,m", [("heisenberg", 24, 11, 1100), ("qc_su2", 10, 4, 131)])
+def test_adjoint_of_groups_side_by_side(model, L, site, m):
+    """Gradients of plans whose groups' products run on the side streams (a context of its own shows them
+    being made: four library handles of at least 32 MiB each beyond what the plan reports), three through
+    one plan, against the oracle: all terms of the spin chain, a sample of the ab initio one."""
+    ws = SyntheticSite(model, L, site, m, seed=L + m)
+    Lc, Rc = ws.random_cohorts(ws.left_index), ws.random_cohorts(ws.right_index)
+    host = host_boundary(ws.left_index, Lc), host_boundary(ws.right_index, Rc)
+    n = ws.mpo_desc.desc.n_terms
+    terms = range(n) if n < 50 else sorted(set(ws.rng.integers(0, n, 40).tolist()))
+    eng = E.Engine(0)
+    try:
+        Lb, Rb = E.DeviceBoundary.upload(eng, ws.left_index, Lc), E.DeviceBoundary.upload(eng, ws.right_index, Rc)
+        torch.cuda.synchronize()
+        free0 = torch.cuda.mem_get_info()[0]
+        plan = E.SigmaPlan(eng, ws.site_desc, ws.mpo_desc, Lb, Rb, algorithm=E.SIGMA_GROUPED, adjoint=True)
+        assert free0 - torch.cuda.mem_get_info()[0] - plan.workspace_bytes >= 128 << 20
+        psis = [ws.random_psi() for _ in range(2)]
+        grads = [plan.adjoint(torch.from_numpy(x).to("cuda:0")) for x in psis + psis[:1]]
+        assert np.array_equal(grads[0], grads[2])
+        for x, g in zip(psis, grads):
+            ref = np.array([float(np.dot(x, O.SigmaOracle(ws.site_desc, O._TermMpo(ws.mpo_desc, t), *host).apply(x)))
+                            for t in terms])
+            err = np.linalg.norm(g[list(terms)] - ref) / np.linalg.norm(ref)
+            print("adjoint %s L=%d site=%d m=%d: %.2e" % (model, L, site, m, err), flush=True)
+            assert err <= 10 * RTOL[E.PREC_F64]   # two products in a row and the sum over a term's entries
+        plan.close()
+    finally:
+        eng.close()
