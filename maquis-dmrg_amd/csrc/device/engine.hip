@@ -2429,7 +2429,8 @@ void add_bsr_groups(StagePlan::Bsr& B, const std::vector<GroupedLowering::Group>
         // of one row panel with every W panel of the group (or the reverse)
         constexpr uint32_t SB = 8;
         const uint32_t npm = (M + TM - 1) / TM;
-        B.narrow = B.narrow && (32ull * M + TM) * sizeof(double) < (1ull << 32);
+        static const bool wide = std::getenv("MQ_S_WIDE") != nullptr;   // tests: 64-bit offsets at any size
+        B.narrow = B.narrow && !wide && (32ull * M + TM) * sizeof(double) < (1ull << 32);
         for (uint32_t jb = 0; jb < npn; jb += SB)
             for (uint32_t mb = 0; mb < npm; mb += SB)
                 for (uint32_t j = jb; j < std::min(npn, jb + SB); ++j)

@@ -369,3 +369,38 @@ def test_adjoint_of_groups_side_by_side(model, L, site, m):
         plan.close()
     finally:
         eng.close()
+
+
+WIDE = """
+import hashlib
+import torch
+from mqdmrg import engine as E
+from mqdmrg.workloads import SyntheticSite
+eng = E.Engine(0)
+for a in [("heisenberg", 16, 7, 150), ("qc", 8, 3, 77), ("qc_su2", 10, 4, 131), ("qc_su2", 14, 6, 101)]:
+    ws = SyntheticSite(*a, seed=3)
+    Lb = E.DeviceBoundary.upload(eng, ws.left_index, ws.random_cohorts(ws.left_index))
+    Rb = E.DeviceBoundary.upload(eng, ws.right_index, ws.random_cohorts(ws.right_index))
+    plan = E.SigmaPlan(eng, ws.site_desc, ws.mpo_desc, Lb, Rb)
+    psi = torch.from_numpy(ws.random_psi()).to("cuda:0")
+    for prec in (E.PREC_F64, E.PREC_F32, E.PREC_BF16X3):
+        out = torch.empty_like(psi)
+        plan.apply(psi, out, precision=prec)
+        eng.sync()
+        print("digest", *a, prec, hashlib.sha256(out.cpu().numpy().tobytes()).hexdigest(), flush=True)
+    plan.close()
+eng.close()
+"""
+
+
+def test_wide_groups_have_the_same_bits():
+    """Groups of 2^24 rows and more address T_D with 64-bit offsets and plain loads: MQ_S_WIDE=1 takes that
+    form at any size, with every bit as with 32-bit offsets (which the oracle tests cover)."""
+    def digests(**env):
+        r = subprocess.run([sys.executable, "-c", WIDE], capture_output=True, text=True, timeout=100,
+                           env=dict(os.environ, PYTHONPATH=os.pathsep.join(sys.path), **env))
+        assert r.returncode == 0, r.stderr[-2000:]
+        return [x for x in r.stdout.splitlines() if x.startswith("digest")]
+
+    narrow = digests()
+    assert len(narrow) == 12 and digests(MQ_S_WIDE="1") == narrow
