@@ -844,7 +844,7 @@ struct StagePlan {
         double* ent_val = nullptr;
         uint64_t n_ent = 0;
         uint64_t tiles = 0;
-        uint64_t flops = 0;             // MFMA flops of the visited tiles (unpadded)
+        uint64_t flops = 0;             // MFMA flops of the visited tiles' blocks with a nonzero (unpadded)
         bool narrow = true;             // every task's T_D step window fits 32-bit byte offsets
         std::vector<uint32_t> tile_cols;   // per tile: the 16-column blocks holding a nonzero (bits)
         // per tile: its group, first key and first column: the dense W_D can be rebuilt from the
@@ -2411,15 +2411,21 @@ void add_bsr_groups(StagePlan::Bsr& B, const std::vector<GroupedLowering::Group>
         MQ_REQUIRE(g.M < (1ull << 32), "group too large for the block-sparse S stage");
         const uint32_t Kg = uint32_t(g.K.size()), Ng = uint32_t(g.N.size()), M = uint32_t(g.M);
         const uint32_t npn = uint32_t(S.panel_runs.size());
-        uint64_t tile = tile0[gi];
+        uint64_t tile = tile0[gi], multiplied = 0;
         std::vector<std::pair<uint32_t, uint32_t>> pr(npn);
         for (uint32_t j = 0; j < npn; ++j) {
             pr[j].first = uint32_t(B.runs.size());
             for (const auto& r : S.panel_runs[j]) {
                 const uint32_t k0 = r.first * TK, k1 = std::min(Kg, (r.first + r.second) * TK);
                 B.runs.push_back({k0, k1 - k0, uint32_t(tile), 0u});
-                for (uint32_t t = 0; t < r.second; ++t)
-                    B.tile_at.push_back({uint32_t(gi), (r.first + t) * TK, j * TN});
+                for (uint32_t t = 0; t < r.second; ++t) {
+                    const uint32_t kt = (r.first + t) * TK, on = B.tile_cols[tile + t];
+                    B.tile_at.push_back({uint32_t(gi), kt, j * TN});
+                    // the columns of its blocks with a nonzero, the group's last block unpadded
+                    uint32_t cols = 16 * uint32_t(__builtin_popcount(on));
+                    if (j + 1 == npn && on >> ((Ng - 1 - j * TN) / 16)) cols -= (16 - Ng % 16) % 16;
+                    multiplied += uint64_t(std::min(Kg - kt, TK)) * cols;
+                }
                 tile += r.second;
             }
             pr[j].second = uint32_t(B.runs.size());
@@ -2440,7 +2446,7 @@ void add_bsr_groups(StagePlan::Bsr& B, const std::vector<GroupedLowering::Group>
                         B.tasks.push_back({g.t_off + m0, g.s_off + uint64_t(n0) * g.M + m0, mr, nw, M, pr[j].first,
                                            pr[j].second, 0u});
                     }
-        B.flops += 2ull * g.M * S.visited;
+        B.flops += 2ull * g.M * multiplied;
     }
     if (g_trace) {
         uint64_t on = 0;
@@ -3976,7 +3982,7 @@ int mq_plan_profile(mq_plan* p, const double* psi, double* sigma, int reps, int 
             ft = gemm_flops(P.t_tasks, P.t_segs);
             ff = gemm_flops(P.f_tasks, P.f_segs);
             P.for_regions([&](const GatherRegion& r) { fg += 2ull * r.R * r.C * (r.t1 - r.t0); });
-            // S stage: the block-sparse kernel's visited tiles, and the dense library GEMMs of the rest
+            // S stage: what the block-sparse kernel multiplies, and the dense library GEMMs of the rest
             for (const auto& g : P.lib)
                 if (!g.sparse) fg += 2ull * g.M * g.N * g.K;
             fg += P.bsr.flops;

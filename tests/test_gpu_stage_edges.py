@@ -404,3 +404,18 @@ def test_wide_groups_have_the_same_bits():
 
     narrow = digests()
     assert len(narrow) == 12 and digests(MQ_S_WIDE="1") == narrow
+
+
+def test_profile_counts_the_products_made(eng):
+    """The S-stage flops that a profile reports are those of the blocks the kernel multiplies: their rate is
+    below the chip's FP64 matrix peak (78.6 TFLOP/s), which the visited tiles counted whole exceed."""
+    ws = SyntheticSite("qc_su2", 24, 11, 700, seed=2)
+    Lb = E.DeviceBoundary.upload(eng, ws.left_index, ws.random_cohorts(ws.left_index))
+    Rb = E.DeviceBoundary.upload(eng, ws.right_index, ws.random_cohorts(ws.right_index))
+    plan = E.SigmaPlan(eng, ws.site_desc, ws.mpo_desc, Lb, Rb)
+    psi = torch.from_numpy(ws.random_psi()).to("cuda:0")
+    ms, flops, _ = plan.profile(psi, torch.empty_like(psi), reps=5)
+    model = plan.flops - flops[0] - flops[2]   # one multiplication per nonzero coupling
+    print("S stage %.3f ms, %.3e flops, %.1f TFLOP/s; couplings %.3e" % (ms[2], flops[1], flops[1] / ms[2] * 1e-9, model), flush=True)
+    assert 0 < model < flops[1] < 78.6e9 * ms[2]
+    plan.close()
