@@ -398,8 +398,8 @@ def main():
     # the reference's model (solver/tasks.cpp:388-398, 777-796) per second: for the T and final stages
     # these are the block products the kernel executes; for the S stage the model counts one alpha
     # per nonzero MPO coupling, i.e. the plan's model flops minus those of the T and final stages
-    # (the executed MFMA flops, which include the zeros inside the visited W_D tiles, are reported
-    # beside it).
+    # (the executed MFMA flops, which include the zeros inside the 16 x 16 blocks of W_D that hold a
+    # nonzero, are reported beside it).
     pr = per[report]
     st = pr["stage_ms"]
     dom = max(["gemm_T", "gemm_S", "gemm_final"], key=lambda k: st[k])
@@ -413,9 +413,10 @@ def main():
             {"f64": "FP64", "f32": "FP32", "bf16x3": "bf16 split-product, FP32 accumulate"}[report])
         peak_key = report
     else:
-        # T and final stages: the lean MFMA kernels (and the generic grouped GEMM for other tile
-        # shapes), FP32 accumulation in the reduced precisions
-        kernel = ("mq::t_stream_kernel (T stage)" if dom == "gemm_T" else "mq::f_unit_kernel (final stage)")
+        # T and final stages: several kernels by task shape, FP32 accumulation in the reduced precisions
+        kernel = ("T stage: mq::t_stream_kernel (K <= 288 and N >= 128), mq::t_stack_kernel, mq::gemm_kernel"
+                  if dom == "gemm_T" else
+                  "final stage: mq::f_unit_kernel, mq::f_wave_kernel (at most 32 rows; small FP64 stages), mq::gemm_kernel")
         peak_key = "f64" if report == "f64" else "f32"
     roof = {"kernel": kernel, "bound": "mfma", "achieved": achieved, "peak": PEAK_TFLOPS[peak_key],
             "unit": "TFLOP/s", "frac": achieved / PEAK_TFLOPS[peak_key], "traffic": None, "stage_ms": st,

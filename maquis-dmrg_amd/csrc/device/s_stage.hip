@@ -10,17 +10,20 @@
 // has rows of its own, and the compact W tiles, which all waves share, through LDS, double buffered.
 //
 // What bounds it: FP64 the MFMA rate (matrix units busy 80% of the time; 61 of the 73 TFLOP/s a large FP64
-// product reaches, counting the zeros inside visited 16 x 16 blocks), BF16X3 the memory (L=30:
-// 31 GB read, T_D about twice, and 8.4 GB written in 8.3 ms, 4.8 TB/s).  A visited 16 x 128 tile is on average two thirds full by 16-column blocks; every wave
-// spans the tile's 128 columns and skips the blocks without a nonzero (the same for every wave; adding a
-// zero product changes no bit), and the loads run two steps ahead.  S stage at SU2U1 L=30 m=1500: FP64
+// product reaches, counting the zeros inside visited 16 x 16 blocks), BF16X3 the memory: at L=30, m=1500
+// it reads 31 GB and writes 8.4 GB in 8.3 ms, 4.8 TB/s, where T_D once is 8.2 GB.  The 8 x 8 panel blocks ask
+// for T_D once per 8 column panels and for W once per 8 row panels, 18 and 5 GB; the rest of what is read
+// comes back because a block's panels do not stay in L2 for all of it.  A visited 16 x 128 tile is on average
+// two thirds full by 16-column blocks; every wave spans the tile's 128 columns and skips the blocks without
+// a nonzero (the same for every wave; adding a zero product of finite values changes no bit), and the loads
+// run two steps ahead.  S stage at SU2U1 L=30 m=1500: FP64
 // 49.8 ms with every block multiplied, 30.8 ms with blocks skipped, tiles dealt to the XCDs and T_D staged
 // through LDS, 26.1 ms with T_D read directly, W read in whole lines and 8 waves; BF16X3 9.3 -> 8.3 ms.
 // L=24 m=1000: FP64 13.3, 7.1, 5.8 ms; BF16X3 2.85, 2.45, 2.2 ms.  Three arithmetics:
 //
 //   MODE_F64     v_mfma_f64_16x16x4f64 on FP64 T_D / W tiles (the plain path)
 //   MODE_F32     v_mfma_f32_16x16x4f32 on FP32 T_D / W tiles
-//   MODE_BF16X3  FP32 T_D split on the fly into bf16 hi + lo while it is staged, W tiles split once
+//   MODE_BF16X3  FP32 T_D split on the fly into bf16 hi + lo in registers, W tiles split once
 //                per plan; three v_mfma_f32_16x16x32_bf16 products per block and 32-key step
 //                (hi*lo + lo*hi + hi*hi) with FP32 accumulation, the split-product scheme of the
 //                library path (gfx950's K = 32 bf16 MFMA: twice the rate per key of the K = 16 form)
