@@ -742,13 +742,16 @@ void step_final_kernel(const GemmTask* __restrict__ tasks, uint32_t n_tasks, con
         }
     };
     auto store = [&](const Stage& s, int buf) {
-        double x[4];
+        double x[4], y[4];   // both zero beyond the segment: 0 times an infinity of its last key would be a NaN
 #pragma unroll
-        for (int e = 0; e < 4; ++e) x[e] = s.k0 + a_k + e < s.K ? s.a[e] * s.sc : 0.0;
+        for (int e = 0; e < 4; ++e) {
+            x[e] = s.k0 + a_k + e < s.K ? s.a[e] * s.sc : 0.0;
+            y[e] = s.k0 + b_k + e < s.K ? s.b[e] : 0.0;
+        }
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             *reinterpret_cast<double2*>(&sa[buf][a_m][a_k + 2 * h]) = double2{x[2 * h], x[2 * h + 1]};
-            *reinterpret_cast<double2*>(&sb[buf][b_n][b_k + 2 * h]) = double2{s.b[2 * h], s.b[2 * h + 1]};
+            *reinterpret_cast<double2*>(&sb[buf][b_n][b_k + 2 * h]) = double2{y[2 * h], y[2 * h + 1]};
         }
     };
     d4 acc[RS_BN / 16];

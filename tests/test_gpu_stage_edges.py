@@ -419,3 +419,37 @@ def test_profile_counts_the_products_made(eng):
     print("S stage %.3f ms, %.3e flops, %.1f TFLOP/s; couplings %.3e" % (ms[2], flops[1], flops[1] / ms[2] * 1e-9, model), flush=True)
     assert 0 < model < flops[1] < 78.6e9 * ms[2]
     plan.close()
+
+
+@pytest.mark.parametrize("kind", ["left", "right"])
+@pytest.mark.parametrize("model,L,site,m", [("heisenberg", 16, 7, 150), ("hubbard", 12, 5, 301)])
+def test_step_keeps_infinities_of_the_bra(eng, kind, model, L, site, m):
+    """An infinity in the bra reaches the elements of the new boundary that it contributes to as an infinity of
+    the oracle's sign, also where it is the last key of a segment that is no multiple of 16 (a NaN if the
+    padding multiplied it).  Elsewhere a zero of S_D may meet it, which the oracle's sum does not hold."""
+    from mqdmrg import mps
+    from mqdmrg.symmetry import SiteLayout
+    ws = SyntheticSite(model, L, site, m, seed=L + m)
+    k = site if kind == "left" else site + 1
+    index = ws.left_index if kind == "left" else ws.right_index
+    lay = SiteLayout(ws.bonds[k], ws.basis.phys, ws.bonds[k + 1])
+    sd, md = E.SiteDesc(ws.basis.sym, ws.bonds[k], ws.basis.phys, ws.bonds[k + 1]), E.MpoDesc(ws.mpo[k])
+    coh = ws.random_cohorts(index)
+    hb = host_boundary(index, coh)
+    bra, ket = mps.random_site_vector(lay, ws.rng), mps.random_site_vector(lay, ws.rng)
+    # the last element of the largest block: last key of its row (left step) or column segment (right step)
+    lb = max(range(len(lay.left.sizes)), key=lambda i: lay.left.sizes[i] * lay.rp_cols[i])
+    bra[lay.rp_offset[lb] + lay.left.sizes[lb] * lay.rp_cols[lb] - 1] = np.inf
+    d = lambda x: torch.from_numpy(np.ascontiguousarray(x)).to("cuda:0")  # noqa: E731
+    b = E.DeviceBoundary.upload(eng, index, coh)
+    if kind == "left":
+        ref = O.left_step(sd, md, mps.rp_to_lp(lay, bra), ket, hb, True)
+        new = E.left_step(eng, sd, md, d(mps.rp_to_lp(lay, bra)), d(ket), b)
+    else:
+        ref = O.right_step(sd, md, bra, ket, hb, True)
+        new = E.right_step(eng, sd, md, d(bra), d(ket), b)
+    got, want = np.concatenate(new.download()), np.concatenate(ref.cohorts)
+    print("%s %s: infinities %d of %d, NaN %d of %d" % (kind, model, np.isinf(got).sum(), np.isinf(want).sum(),
+                                                       np.isnan(got).sum(), np.isnan(want).sum()), flush=True)
+    assert np.isinf(want).any()
+    assert np.array_equal(np.isposinf(got), np.isposinf(want)) and np.array_equal(np.isneginf(got), np.isneginf(want))
