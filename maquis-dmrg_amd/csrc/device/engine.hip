@@ -844,13 +844,27 @@ struct StagePlan {
         double* ent_val = nullptr;
         uint64_t n_ent = 0;
         uint64_t tiles = 0;
-        uint64_t flops = 0;             // MFMA flops of the visited tiles' blocks with a nonzero (unpadded)
         bool narrow = true;             // every task's T_D step window fits 32-bit byte offsets
         std::vector<uint32_t> tile_cols;   // per tile: the 16-column blocks holding a nonzero (bits)
         // per tile: its group, first key and first column: the dense W_D can be rebuilt from the
         // tiles (the flop model reads W_D; the device keeps only the tiles)
         struct TileAt { uint32_t group, k0, n0; };
         std::vector<TileAt> tile_at;
+        struct GroupAt { uint64_t M; uint32_t K, N; };
+        std::vector<GroupAt> group_at;
+        // MFMA flops of the visited tiles' 16-column blocks with a nonzero (unpadded)
+        uint64_t flops() const {
+            uint64_t f = 0;
+            for (size_t i = 0; i < tile_at.size(); ++i) {
+                const TileAt& t = tile_at[i];
+                const GroupAt& g = group_at[t.group];
+                uint64_t cols = 0;
+                for (uint32_t n = t.n0, on = tile_cols[i]; on; n += 16, on >>= 1)
+                    if (on & 1) cols += std::min(g.N - n, 16u);
+                f += 2 * g.M * std::min<uint32_t>(g.K - t.k0, S_BSR_TILE_K) * cols;
+            }
+            return f;
+        }
         DevBuf d_tasks, d_runs, d_tile_cols, d_w64, d_w32, d_whi, d_wlo;
     } bsr;
     bool bsr_on = false;
@@ -2404,6 +2418,7 @@ void add_bsr_groups(StagePlan::Bsr& B, const std::vector<GroupedLowering::Group>
     // runs and tasks in group order
     for (size_t gi = 0; gi < ng; ++gi) {
         const auto& g = groups[gi];
+        B.group_at.push_back({g.M, uint32_t(g.K.size()), uint32_t(g.N.size())});
         const BsrGroupScan& S = sc[gi];
         if (info) info->push_back({S.nnz, g.K.empty() || g.N.empty() ? 0.0 :
                                               double(S.visited) / (double(g.K.size()) * double(g.N.size()))});
@@ -2411,21 +2426,15 @@ void add_bsr_groups(StagePlan::Bsr& B, const std::vector<GroupedLowering::Group>
         MQ_REQUIRE(g.M < (1ull << 32), "group too large for the block-sparse S stage");
         const uint32_t Kg = uint32_t(g.K.size()), Ng = uint32_t(g.N.size()), M = uint32_t(g.M);
         const uint32_t npn = uint32_t(S.panel_runs.size());
-        uint64_t tile = tile0[gi], multiplied = 0;
+        uint64_t tile = tile0[gi];
         std::vector<std::pair<uint32_t, uint32_t>> pr(npn);
         for (uint32_t j = 0; j < npn; ++j) {
             pr[j].first = uint32_t(B.runs.size());
             for (const auto& r : S.panel_runs[j]) {
                 const uint32_t k0 = r.first * TK, k1 = std::min(Kg, (r.first + r.second) * TK);
                 B.runs.push_back({k0, k1 - k0, uint32_t(tile), 0u});
-                for (uint32_t t = 0; t < r.second; ++t) {
-                    const uint32_t kt = (r.first + t) * TK, on = B.tile_cols[tile + t];
-                    B.tile_at.push_back({uint32_t(gi), kt, j * TN});
-                    // the columns of its blocks with a nonzero, the group's last block unpadded
-                    uint32_t cols = 16 * uint32_t(__builtin_popcount(on));
-                    if (j + 1 == npn && on >> ((Ng - 1 - j * TN) / 16)) cols -= (16 - Ng % 16) % 16;
-                    multiplied += uint64_t(std::min(Kg - kt, TK)) * cols;
-                }
+                for (uint32_t t = 0; t < r.second; ++t)
+                    B.tile_at.push_back({uint32_t(gi), (r.first + t) * TK, j * TN});
                 tile += r.second;
             }
             pr[j].second = uint32_t(B.runs.size());
@@ -2446,7 +2455,6 @@ void add_bsr_groups(StagePlan::Bsr& B, const std::vector<GroupedLowering::Group>
                         B.tasks.push_back({g.t_off + m0, g.s_off + uint64_t(n0) * g.M + m0, mr, nw, M, pr[j].first,
                                            pr[j].second, 0u});
                     }
-        B.flops += 2ull * g.M * multiplied;
     }
     if (g_trace) {
         uint64_t on = 0;
@@ -3985,7 +3993,7 @@ int mq_plan_profile(mq_plan* p, const double* psi, double* sigma, int reps, int 
             // S stage: what the block-sparse kernel multiplies, and the dense library GEMMs of the rest
             for (const auto& g : P.lib)
                 if (!g.sparse) fg += 2ull * g.M * g.N * g.K;
-            fg += P.bsr.flops;
+            fg += P.bsr.flops();
             flops_out[0] = ft;
             flops_out[1] = fg;
             flops_out[2] = ff;
