@@ -742,11 +742,15 @@ void step_final_kernel(const GemmTask* __restrict__ tasks, uint32_t n_tasks, con
         }
     };
     auto store = [&](const Stage& s, int buf) {
-        double x[4], y[4];   // both zero beyond the segment: 0 times an infinity of its last key would be a NaN
+        double x[4], y[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            x[e] = s.k0 + a_k + e < s.K ? s.a[e] * s.sc : 0.0;
-            y[e] = s.k0 + b_k + e < s.K ? s.b[e] : 0.0;
+        for (int e = 0; e < 4; ++e) x[e] = s.a[e] * s.sc, y[e] = s.b[e];
+        if (s.k0 + TK > s.K) {   // keys beyond the segment: both zero (0 times an infinity of its last key is a NaN)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if (s.k0 + a_k + e >= s.K) x[e] = 0.0;
+                if (s.k0 + b_k + e >= s.K) y[e] = 0.0;
+            }
         }
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
