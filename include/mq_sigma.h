@@ -326,8 +326,8 @@ int mq_sigma_apply_batched(mq_ctx* ctx, int n, mq_plan* const* plans, const doub
 /* Measurement: runs `reps` sigma applications stage by stage with HIP events on the context's
  * stream and returns the average milliseconds of each stage: [0] S zero-fill, [1] T-stage GEMM,
  * [2] S gather, [3] final GEMM.  flops_out (may be NULL) receives the algorithmic flops of the
- * three compute stages (T GEMM, gather, final GEMM) and gather_bytes (may be NULL) the
- * algorithmic bytes of the gather (T slab reads + S writes). */
+ * three compute stages (T GEMM, gather, final GEMM; the block-sparse S stage: the products it makes)
+ * and gather_bytes (may be NULL) the algorithmic bytes of the gather (T slab reads + S writes). */
 int mq_plan_profile(mq_plan* plan, const double* psi, double* sigma, int reps, int precision,
                     double* stage_ms, uint64_t* flops_out, uint64_t* gather_bytes);
 int mq_plan_vector_size(const mq_plan* plan, uint64_t* n_elements);
